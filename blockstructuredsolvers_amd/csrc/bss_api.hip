@@ -127,7 +127,6 @@ struct bss_plan {
   std::vector<int> chain_len = std::vector<int>(16, 0);  // per-level overrides
   int chain_len_default = 3;
   int base_max = 8;
-  int factor_waves = 4;
   bool preserve = true;  // plain mode: factors to workspace, A/B untouched
   // bss_info: per-system LAPACK-order info of the last factorisation, computed once
   std::vector<int> info_exact;
@@ -646,9 +645,9 @@ int factor_levels(bss_plan* p, hipStream_t s, size_t l_begin = 0, size_t l_end =
     {
       ProfScope ps(p, BSS_K_FACTOR, (int)l, s);
       if (l == 0)
-        e = bss::launch_factor<Tin, T>(nb, p->factor_waves, a, (int)G.chains.size(), s);
+        e = bss::launch_factor<Tin, T>(nb, a, (int)G.chains.size(), s);
       else
-        e = bss::launch_factor<T, T>(nb, p->factor_waves, a, (int)G.chains.size(), s);
+        e = bss::launch_factor<T, T>(nb, a, (int)G.chains.size(), s);
     }
     if (e != hipSuccess) return fail(BSS_E_HIP, "factor level %zu launch: %s", l, hipGetErrorString(e));
     if (!G.seps.empty()) {
@@ -677,7 +676,7 @@ int refactor_separators64(bss_plan* p, hipStream_t s) {
     const bss::FactorLevelArgs a{G.dchains, G.dtab64[0], p->dinfo, nullptr};
     {
       ProfScope ps(p, BSS_K_FACTOR, (int)l, s);
-      e = bss::launch_factor<double, double>(nb, p->factor_waves, a, (int)G.chains.size(), s);
+      e = bss::launch_factor<double, double>(nb, a, (int)G.chains.size(), s);
     }
     if (e == hipSuccess && !G.seps.empty()) {
       ProfScope ps(p, BSS_K_ASSEMBLE_DIAG, (int)l, s);
@@ -926,7 +925,6 @@ int fallback_solve(bss_plan* p, hipStream_t s) {
     q->chain_len = p->chain_len;
     q->chain_len_default = p->chain_len_default;
     q->base_max = p->base_max;
-    q->factor_waves = p->factor_waves;
     q->preserve = true;
     if (int e = bss_plan_bind(q, p->A, p->B, x0)) {
       bss_plan_destroy(q);
@@ -1158,7 +1156,6 @@ int bss_set_option(bss_plan_t p, int option, double value) {
       return BSS_OK;
     case BSS_OPT_FACTOR_WAVES:
       if (value != 4 && value != 8) return fail(BSS_E_ARG, "factor waves must be 4 or 8");
-      p->factor_waves = (int)value;
       p->drop_graphs();
       return BSS_OK;
     case BSS_OPT_GRAPH:

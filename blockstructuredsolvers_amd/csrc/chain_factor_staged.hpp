@@ -1,10 +1,10 @@
-// chain_factor_staged.hpp -- chain factorisation for block sizes n = 96 and 128.
+// chain_factor_staged.hpp -- chain factorisation of FP64 factors at block size n = 128.
 //
-// Same algorithm and outputs as chain_factor_kernel (chain_factor.hpp): per chain
+// Same algorithm and outputs as chain_factor_strip_kernel: per chain
 //   Z_s = B_L^T,  for each block i:  A_i -= C_{i-1}^T C_{i-1};  Uinv_i = chol(A_i)^{-1};
 //   [C_i | W_i] = Uinv_i^T [B_i | Z_i];  Z_{i+1} = -C_i^T W_i;  S_L += W_i^T W_i
-// but at these sizes four n x n blocks no longer fit in the 160 KB of LDS (one FP64
-// block at n = 128 is 128 KB).  Only the upper triangle of the block being factored
+// but one FP64 block at n = 128 is 128 KB, and the strip kernel's LDS (a triangle and a
+// block) would exceed the 160 KB of a CU.  Only the upper triangle of the block being factored
 // stays in LDS, as packed 16x16 tiles; it is factored in place (potrf, diagonal tiles
 // kept inverted) and then inverted in place (trtri), giving Uinv.  B, Z and the
 // products C, W live in their HBM output slots and reach the MFMAs through two LDS
@@ -107,44 +107,20 @@ __device__ inline void gtile_store(BSS_GLOBAL T* p, int ld, const typename Mfma<
 // (put(regs, buf)) and multiplied after one barrier (mul(s, buf)).  When a wave passes
 // the barrier of step s, every wave has finished mul(s - 1), so buffer (s + 1) & 1 is
 // free for the next put.  The closing barrier leaves both buffers free.
-// With one buffer (NBUF = 1) a second barrier per step waits for every mul(s - 1)
-// before the buffer is overwritten.
-template <typename Regs, int NBUF, typename Load, typename Put, typename Mul>
+template <typename Regs, typename Load, typename Put, typename Mul>
 __device__ __attribute__((always_inline)) inline void staged_steps(int steps, Load&& load,
                                                                    Put&& put, Mul&& mul) {
   Regs r;
   if (steps > 0) load(0, r);
-  auto step = [&](int s) {
-    const int buf = NBUF == 1 ? 0 : (s & 1);
-    if (NBUF == 1 && s > 0) __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    const int buf = s & 1;
     put(r, buf);
     __syncthreads();
     if (s + 1 < steps) load(s + 1, r);
     mul(s, buf);
-  };
-  if constexpr (NBUF == 1) {
-    // the single-buffered variants run at 128 registers a wave: an unrolled step loop
-    // spills inside the steps (28.9 against 31.2 ms for the level-0 FP32 factorisation
-    // of 16 systems at n = 128)
-#pragma unroll 1
-    for (int s = 0; s < steps; ++s) step(s);
-  } else {
-    for (int s = 0; s < steps; ++s) step(s);
   }
   __syncthreads();
 }
-
-// Staging buffers and workgroups per CU.  FP32 factors single-buffer (66 KB of LDS at
-// n = 128) so that two workgroups share a CU and one's potrf and trtri overlap the
-// other's products, within 128 registers a wave (level-0 factorisation of 16 systems
-// at n = 128: 28.9 ms against 37.2 ms with one double-buffered workgroup per CU).  FP64
-// factors double-buffer with one workgroup per CU: at n = 96 two workgroups would fit
-// in LDS, but the 128-register cap spills (41.1 ms against 34.0 ms).
-template <typename T, int NB>
-struct StagedCfg {
-  static constexpr int NBUF = sizeof(T) == 4 ? 1 : 2;
-  static constexpr int WG_PER_CU = NBUF == 2 ? 1 : 2;
-};
 
 // Quads per thread of one staged operand: a 16-row slice (4 quads per column) of an
 // n-column block, or a pair of 16-column panels (n / 4 quads per column)
@@ -162,7 +138,7 @@ struct QuadRegs {
 };
 
 template <typename Tin, typename T, int NB, int NW>
-__global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4))
+__global__ void __launch_bounds__(64 * NW, NW / 4)
     chain_factor_staged_kernel(FactorLevelArgs p) {
   typedef StagedTri<T, NB> Tri;
   constexpr int TT = Tri::TT, NS = Tri::NS, LDT = Tri::LDT, TS = Tri::TS;
@@ -178,8 +154,7 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
   typedef typename Mfma<T>::acc_t acc_t;
 
   __shared__ __attribute__((aligned(16))) T tri[NS * TS];
-  constexpr int NBUF = StagedCfg<T, NB>::NBUF;
-  __shared__ __attribute__((aligned(16))) T stg[NBUF * 2 * OP];  // buffers x 2 operands
+  __shared__ __attribute__((aligned(16))) T stg[2 * 2 * OP];  // buffers x 2 operands
   __shared__ int fail;
 
   const ChainRec cd = p.chains[blockIdx.x];
@@ -243,8 +218,7 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
 #pragma unroll
   for (int q = 0; q < SQ; ++q) Sacc[q] = Mfma<T>::zero();
   if (tid == 0) fail = 0;
-  int fail_i = len;      // first failed block of the chain (thread 0)
-  float piv_run = 1.0f;  // smallest pivot ratio of the chain (wave 0)
+  int fail_i = len;  // first failed block of the chain (thread 0)
 
   if (hasL) {  // Z_1 = B_L^T into the first block's panel slot
     const BSS_GLOBAL Tin* bl = B + (long long)(start - 1) * NN;
@@ -277,7 +251,7 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
       }
       if (i > 0) {
         const BSS_GLOBAL T* Cp = C + (blk - 1) * NN;
-        staged_steps<QuadRegs<T, Sh::SLICE_QPT>, NBUF>(
+        staged_steps<QuadRegs<T, Sh::SLICE_QPT>>(
             TT, [&](int kt, auto& r) { slice_load(r.v, Cp, kt); },
             [&](const auto& r, int buf) { slice_put(stg + buf * 2 * OP, r.v); },
             [&](int kt, int buf) {
@@ -304,14 +278,6 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
       }
     }
     __syncthreads();  // triangle complete
-    float adiag[2] = {0.0f, 0.0f};
-    if (p.pivmin && w == 0) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int j = lane_id() + 64 * h;
-        if (j < NB) adiag[h] = (float)tri[Tri::idx(j >> 4, j >> 4) + (j & 15) * (LDT + 1)];
-      }
-    }
     // 2. potrf in place: diagonal tiles become Uinv_kk, row panels U_kj.  Lookahead:
     //    during the trailing update of step kk, wave 0 updates tile (kk+1, kk+1) first
     //    (task 0) and factors it at once while the other waves share the remaining
@@ -349,25 +315,11 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
         __syncthreads();
       }
     }
-    // reported once after the chain (see chain_factor.hpp)
+    // reported once after the chain: a global atomic inside the loop, on a path some lanes
+    // skip, would make the memory waits after it conservative
     if (tid == 0 && fail) {
       fail_i = min(fail_i, i);
       fail = 0;
-    }
-    if (p.pivmin && w == 0) {
-      float ratio = 1.0f;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int j = lane_id() + 64 * h;
-        if (j < NB) {
-          const float ui = (float)tri[Tri::idx(j >> 4, j >> 4) + (j & 15) * (LDT + 1)];
-          const float q = 1.0f / (ui * ui * adiag[h]);
-          ratio = fminf(ratio, (q >= 0.0f && q <= 3.0e38f) ? q : 0.0f);
-        }
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) ratio = fminf(ratio, __shfl_xor(ratio, o));
-      piv_run = fminf(piv_run, ratio);
     }
     // 3. trtri in place, column by column: Uinv(0:j, j) = -Uinv(0:j, 0:j) U(0:j, j) Uinv_jj
     for (int j = 1; j < TT; ++j) {
@@ -416,13 +368,13 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
     };
     if (hasC) {
       const BSS_GLOBAL Tin* Bb = B + blk * NN;
-      staged_steps<QuadRegs<Tin, Sh::PANEL_QPT>, NBUF>(
+      staged_steps<QuadRegs<Tin, Sh::PANEL_QPT>>(
           TT / 2, [&](int pair, auto& r) { panel_load(r.v, Bb, 32 * pair); },
           [&](const auto& r, int buf) { panel_put(stg + buf * 2 * OP, r.v); },
           [&](int pair, int buf) { solve_mul(Cb, pair, buf); });
     }
     if (hasL) {
-      staged_steps<QuadRegs<T, Sh::PANEL_QPT>, NBUF>(
+      staged_steps<QuadRegs<T, Sh::PANEL_QPT>>(
           TT / 2, [&](int pair, auto& r) { panel_load(r.v, Wb, 32 * pair); },
           [&](const auto& r, int buf) { panel_put(stg + buf * 2 * OP, r.v); },
           [&](int pair, int buf) { solve_mul(Wb, pair, buf); });
@@ -433,7 +385,7 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
       acc_t Z[ZQ];
 #pragma unroll
       for (int q = 0; q < ZQ; ++q) Z[q] = Mfma<T>::zero();
-      staged_steps<QuadRegs<T, 2 * Sh::SLICE_QPT>, NBUF>(
+      staged_steps<QuadRegs<T, 2 * Sh::SLICE_QPT>>(
           TT,
           [&](int kt, auto& r) {
             slice_load(*(T(*)[Sh::SLICE_QPT][4])r.v, Cb, kt);
@@ -480,7 +432,7 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
       for (int q = 0; q < SQ; ++q) R[q] = Mfma<T>::zero();
 #pragma unroll
       for (int q = 0; q < ZQ; ++q) Bp[q] = Mfma<T>::zero();
-      staged_steps<QuadRegs<T, 2 * Sh::SLICE_QPT>, NBUF>(
+      staged_steps<QuadRegs<T, 2 * Sh::SLICE_QPT>>(
           TT,
           [&](int kt, auto& r) {
             if (hasR) slice_load(*(T(*)[Sh::SLICE_QPT][4])r.v, Cb, kt);
@@ -559,7 +511,6 @@ __global__ void __launch_bounds__(64 * NW, (StagedCfg<T, NB>::WG_PER_CU * NW / 4
     const long long blk = start + fail_i;
     atomicMin(p.info + sys, (S.orig ? S.orig[blk] : (int)blk) + 1);
   }
-  if (p.pivmin && tid == 0) atomicMin(p.pivmin + sys, __float_as_uint(piv_run));
 }
 
 }  // namespace bss

@@ -4,75 +4,48 @@
 
 #include "launch.hpp"
 #include "chain_factor_staged.hpp"
+#include "chain_factor_strip.hpp"
 #include "level_kernels.hpp"
 
 namespace bss {
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    cached[dev] = cus;
+template <typename Tin, typename T, int NB>
+static hipError_t factor_strip(const FactorLevelArgs& a, int nchains, hipStream_t s) {
+  if (a.fwd) {  // fused forward sweep: see factor_fuses_forward
+    if constexpr (sizeof(T) == 4 && NB <= 96)
+      hipLaunchKernelGGL((chain_factor_strip_kernel<Tin, T, NB, true>), dim3(nchains),
+                         dim3(4 * NB), 0, s, a);
+    else
+      return hipErrorInvalidValue;
+  } else {
+    hipLaunchKernelGGL((chain_factor_strip_kernel<Tin, T, NB>), dim3(nchains), dim3(4 * NB), 0, s,
+                       a);
   }
-  return cached[dev];
-}
-
-template <typename Tin, typename T, int NB, int NW, bool FWD>
-static hipError_t factor_nb_f(const FactorLevelArgs& a, int nchains, hipStream_t s) {
-  if constexpr (factor_has_latency_variant<T, NB, NW>()) {
-    if (nchains <= device_cus()) {  // one chain per CU at most: latency variant
-      hipLaunchKernelGGL((chain_factor_kernel<Tin, T, NB, NW, true, FWD>), dim3(nchains),
-                         dim3(64 * NW), 0, s, a);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((chain_factor_kernel<Tin, T, NB, NW, false, FWD>), dim3(nchains),
-                     dim3(64 * NW), 0, s, a);
   return hipGetLastError();
 }
 
-template <typename Tin, typename T, int NB, int NW>
-static hipError_t factor_nb(const FactorLevelArgs& a, int nchains, hipStream_t s) {
-  if (a.fwd) {  // fused forward sweep: FP32 factors only (factor_fuses_forward)
-    if constexpr (sizeof(T) == 4)
-      return factor_nb_f<Tin, T, NB, NW, true>(a, nchains, s);
-    else
-      return hipErrorInvalidValue;
-  }
-  return factor_nb_f<Tin, T, NB, NW, false>(a, nchains, s);
-}
-
-template <typename Tin, typename T, int NB, int NW>
-static hipError_t factor_big_nb(const FactorLevelArgs& a, int nchains, hipStream_t s) {
-  if (a.fwd) return hipErrorInvalidValue;  // no fused forward sweep (factor_fuses_forward)
-  hipLaunchKernelGGL((chain_factor_staged_kernel<Tin, T, NB, NW>), dim3(nchains), dim3(64 * NW), 0, s, a);
+// FP64 factors at n = 128 (no pivot monitor: only FP32 levels are monitored)
+static inline hipError_t factor_staged128(const FactorLevelArgs& a, int nchains, hipStream_t s) {
+  if (a.fwd || a.pivmin) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((chain_factor_staged_kernel<double, double, 128, 8>), dim3(nchains),
+                     dim3(512), 0, s, a);
   return hipGetLastError();
 }
 
 template <typename Tin, typename T>
-hipError_t launch_factor(int nb, int waves, const FactorLevelArgs& a, int nchains, hipStream_t s) {
+hipError_t launch_factor(int nb, const FactorLevelArgs& a, int nchains, hipStream_t s) {
   if (nchains <= 0) return hipSuccess;
   switch (nb) {
-    case 16: return factor_nb<Tin, T, 16, 1>(a, nchains, s);
-    case 32: return factor_nb<Tin, T, 32, 2>(a, nchains, s);
-    case 48: return factor_nb<Tin, T, 48, 3>(a, nchains, s);
-    case 64:
-      if (waves == 8) return factor_nb<Tin, T, 64, 8>(a, nchains, s);
-      return factor_nb<Tin, T, 64, 4>(a, nchains, s);
-    case 96:
-      // FP32 factors at n = 96: the four blocks of the LDS kernel fit (154 KB, one
-      // workgroup per CU); FP64 ones take the staged kernel (triangle in LDS)
+    case 16: return factor_strip<Tin, T, 16>(a, nchains, s);
+    case 32: return factor_strip<Tin, T, 32>(a, nchains, s);
+    case 48: return factor_strip<Tin, T, 48>(a, nchains, s);
+    case 64: return factor_strip<Tin, T, 64>(a, nchains, s);
+    case 96: return factor_strip<Tin, T, 96>(a, nchains, s);
+    case 128:  // the strip kernel's LDS: 132 KB with FP32 factors, 262 KB with FP64
       if constexpr (sizeof(T) == 4)
-        return factor_nb<Tin, T, 96, 12>(a, nchains, s);
+        return factor_strip<Tin, T, 128>(a, nchains, s);
       else
-        return factor_big_nb<Tin, T, 96, 8>(a, nchains, s);
-    case 128: return factor_big_nb<Tin, T, 128, 8>(a, nchains, s);
+        return factor_staged128(a, nchains, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -3,7 +3,7 @@
 // the FP32 <-> FP64 hand-off kernels used once separator levels run in FP64.
 #include "kernels_impl.hpp"
 namespace bss {
-template hipError_t launch_factor<double, float>(int, int, const FactorLevelArgs&, int, hipStream_t);
+template hipError_t launch_factor<double, float>(int, const FactorLevelArgs&, int, hipStream_t);
 template hipError_t launch_assemble_diag<double, float, float>(const SepRec*, const LevelSys*, int, int, hipStream_t);
 template hipError_t launch_assemble_diag<double, float, double>(const SepRec*, const LevelSys*, int, int, hipStream_t);
 template hipError_t launch_assemble_rhs<float, double>(const SepRec*, const LevelSys*, int, int, hipStream_t);

@@ -9,10 +9,9 @@
 
 namespace bss {
 
-// `waves`: workgroup size in waves for nb = 64 (4 or 8); other sizes use nb/16.
 // All launchers return hipErrorInvalidValue for an unsupported block size.
 template <typename Tin, typename T>
-hipError_t launch_factor(int nb, int waves, const FactorLevelArgs& a, int nchains, hipStream_t s);
+hipError_t launch_factor(int nb, const FactorLevelArgs& a, int nchains, hipStream_t s);
 template <typename T>
 hipError_t launch_forward(int nb, const SolveLevelArgs& a, int nchains, hipStream_t s);
 template <typename T>

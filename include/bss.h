@@ -98,7 +98,8 @@ enum bss_option {
                                is a failing block of the solver's own elimination order,
                                not necessarily the smallest one LAPACK order gives (the
                                input the sequential re-check needs is gone) */
-  BSS_OPT_FACTOR_WAVES = 6,  /* waves per factor workgroup at n = 64: 4 (default) or 8 */
+  BSS_OPT_FACTOR_WAVES = 6,  /* 4 (default) or 8: accepted, without effect (the factor
+                               kernel's workgroup size follows from n) */
   BSS_OPT_GRAPH = 7,         /* 1 = capture each launch sequence (factorize; solve; in
                                mixed mode each FP32 correction solve) into a hipGraph on
                                first use and replay it afterwards (default 0).  Ignored
