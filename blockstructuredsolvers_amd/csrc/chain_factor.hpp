@@ -1,5 +1,5 @@
 // chain_factor.hpp -- fused per-chain factorisation of one recursion level: the algorithm
-// and the pieces its two kernels share (chain_factor_strip.hpp; chain_factor_staged.hpp
+// and the pieces its two kernels share (chain_factor_strip.hpp; chain_factor_halves.hpp
 // for FP64 factors at n = 128).
 //
 // A level holds N diagonal blocks A_i and N-1 couplings B_i (M = tridiag(B^T, A, B)).
@@ -156,7 +156,8 @@ __device__ __attribute__((always_inline)) inline void diag_step(T (&a)[16], T (&
   if constexpr (J < 15) diag_step<T, J + 1>(a, e, s_next, ok);
 }
 
-// Wave-level Cholesky + inverse of one 16x16 SPD tile held (upper triangle) in LDS.
+// Wave-level Cholesky + inverse of one 16x16 SPD tile held (upper triangle) in LDS, with A
+// and E in separate registers (the probe of tests/gpu_probe; the kernels use diag_img).
 // Row operations are applied to [A | I]; at the end the right half is E = U^{-T}.
 // Writes Uinv = E^T into the upper triangle of the output tile (strict lower part
 // exact zeros).  Returns false if a pivot was not positive.

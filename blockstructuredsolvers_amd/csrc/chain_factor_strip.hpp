@@ -58,9 +58,7 @@ struct Img {
     else
       return 128 * (r >> 3) + 2 * slot(c, (r & 7) >> 1) + (r & 1);
   }
-  // this lane's slots: its own, its A operand's, and for HBM stores (lane l: column l / 4,
-  // vector l % 4, so that four lanes write 64 contiguous bytes; with column l % 16 a store
-  // takes three times as long)
+  // this lane's slots: its own and its A operand's
   __device__ static inline int own_slot() { return slot(lane_id() & 15, lane_id() >> 4); }
   // the column whose vectors are this lane's A operand
   __device__ static inline int a_col() {
@@ -68,7 +66,6 @@ struct Img {
     return sizeof(T) == 4 ? i : (i & 8) + 2 * (i & 3) + ((i >> 2) & 1);
   }
   __device__ static inline int a_slot() { return slot(a_col(), lane_id() >> 4); }
-  __device__ static inline int st_slot() { return slot(lane_id() >> 2, lane_id() & 3); }
   __device__ static inline tile_t load(const T* p, int slot) {
     if constexpr (sizeof(T) == 4) {
       return *(const vec_t*)(p + 4 * slot);
@@ -86,6 +83,14 @@ struct Img {
     }
   }
 };
+
+// The tiles get no defined value but count as written: ends their live range where every
+// later use is behind a write that the compiler cannot see to be always taken.
+template <typename V, int N>
+__device__ __attribute__((always_inline)) inline void forget(V (&t)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) asm volatile("" : "=v"(t[k]));
+}
 
 // acc += X^T Y over one 16-deep step, X as A operand, Y in P layout
 template <typename T>
@@ -293,6 +298,131 @@ __device__ __attribute__((always_inline)) inline bool diag_img(const T* at, T* u
   return __builtin_amdgcn_ballot_w64(!(pv > T(0))) == 0;
 }
 
+// N tiles, one below the other, from consecutive images in LDS to HBM (column-major, leading
+// dimension NB), negated if NEG.  Lane l takes column l / 4, vector l % 4: four lanes write
+// 64 contiguous bytes.  A store from the registers' own lane order (column l % 16) takes 64
+// cycles instead of 20 (1 KB, one CU).  The lane's addresses are formed once: beside the
+// MFMAs of the SIMD's other waves every vector instruction waits for one of them.
+template <typename T, int NB, int N, bool NEG = false>
+__device__ __attribute__((always_inline)) inline void put_tiles(BSS_GLOBAL T* g, const T* tiles) {
+  typedef Img<T> I;
+  typedef typename I::vec_t vec_t;
+  const int l = opaque_v(lane_id());
+  const unsigned off = (unsigned)opaque_v(((l >> 2) * NB + I::VEC * (l & 3)) * (int)sizeof(T));
+  const T* src = tiles + I::VEC * I::slot(l >> 2, l & 3);
+#pragma unroll
+  for (int t = 0; t < N; ++t)
+#pragma unroll
+    for (int h = 0; h < I::PLANES; ++h) {
+      const vec_t x = *(const vec_t*)(src + I::SIZE * t + 128 * h);
+      *(BSS_GLOBAL vec_t*)((BSS_GLOBAL char*)(g + 16 * t + 8 * h) + off) = NEG ? -x : x;
+    }
+}
+
+// potrf and inverse of the n x n block whose upper tiles are in As (packed by columns), by
+// the workgroup's n/16 waves; on return they hold Uinv = U^-1, and so does HBM.  Ls: tiles
+// E(i, t), t < i, of E = U^-T; Es: diagonal tiles of E, two in turn (the first is written
+// while other waves may still read what shares Ls's memory); Is: the identity.
+//
+// Windows k = -1 .. TT-1, one barrier each (the last one the caller's).  In window
+// k < TT-1 wave k+1 updates diagonal tile k+1 with row k and factors it.  The other waves
+// use Uinv_kk, published by window k-1: row i > k takes A(i, j) -= U_ki^T U_kj and
+// E(i, t) -= U_ki^T E_kt, one row a wave, and the waves left over finish Uinv(t, k).  Every
+// wave forms the tiles of row k that it needs itself (U_kj = Uinv_kk^T A_kj), so that row
+// k is never rewritten and one barrier per diagonal tile is enough; with a row-scaling
+// phase and its barrier the FP64 factorisation at n = 64 took 13.6 ms where it takes 12.2.
+// `extra(k)` is the caller's own work in window k.
+template <typename T, int NB>
+struct TileInverse {
+  typedef Img<T> I;
+  typedef typename I::tile_t tile_t;
+  static constexpr int TT = NB / 16, TS = I::SIZE;
+  T *As, *Ls, *Es;
+  const T* Is;
+  int* fail;
+  int w, so, sa;
+
+  __device__ inline T* up(int r, int c) const { return As + (c * (c + 1) / 2 + r) * TS; }
+  __device__ inline T* lo(int i, int t) const { return Ls + (i * (i - 1) / 2 + t) * TS; }
+  __device__ inline T* ed(int k) const { return Es + (k & 1) * TS; }
+
+  // Uinv(u, k) = (Uinv_kk^T E(k, u))^T, to LDS and HBM
+  __device__ __attribute__((always_inline)) inline void finish(BSS_GLOBAL T* U, int u, int k,
+                                                               const tile_t& x) const {
+    tile_t e = Mfma<T>::zero();
+    mma16<T>(e, x, I::load(lo(k, u), so));
+    const auto g = U + 16 * k * NB + 16 * u;
+    const int olr = opaque_v(lane_id() & 15), olk = opaque_v(lane_id() >> 4);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      up(u, k)[I::off(olr, I::row(olk, v))] = e[v];
+      *gat<T>(g + I::row(0, v) * NB, I::row(olk, 0) * NB + olr) = e[v];
+    }
+  }
+  __device__ __attribute__((always_inline)) inline void put_diag(BSS_GLOBAL T* U, int k) const {
+    put_tiles<T, NB, 1>(U + 16 * k * NB + 16 * k, up(k, k));
+  }
+
+  template <typename Extra>
+  __device__ __attribute__((always_inline)) inline void windows(BSS_GLOBAL T* U, Extra extra) const {
+#pragma unroll 1
+    for (int k = -1; k < TT - 1; ++k) {
+      if (w == k + 1) {
+        if (k >= 0) {
+          const tile_t x = I::load(up(k, k), sa);
+          tile_t ub = Mfma<T>::zero(), acc = I::load(up(w, w), so);
+          mma16<T>(ub, x, I::load(up(k, w), so));
+          if constexpr (sizeof(T) == 4) {
+            mma16<T>(acc, -ub, ub);
+          } else {
+            tile_t ua = Mfma<T>::zero();
+            mma16<T>(ua, x, I::load(up(k, w), sa));
+            mma16<T>(acc, -ua, ub);
+          }
+          I::store(up(w, w), so, acc);
+        }
+        if (!diag_img<T>(up(w, w), up(w, w), ed(w), Is) && lane_id() == 0) *fail = 1;
+      } else if (k >= 0) {
+        const tile_t x = I::load(up(k, k), sa);
+        const int u = w - (w > k + 1 ? 1 : 0);
+        if (u < k) {
+          finish(U, u, k, x);
+        } else {
+          const int r = u + 1;  // row r > k
+          tile_t ua = Mfma<T>::zero();
+          mma16<T>(ua, x, I::load(up(k, r), sa));
+          ua = -ua;
+          for (int j = (r == k + 1 ? r + 1 : r); j < TT; ++j) {
+            tile_t ub = Mfma<T>::zero(), acc = I::load(up(r, j), so);
+            mma16<T>(ub, x, I::load(up(k, j), so));
+            mma16<T>(acc, ua, ub);
+            I::store(up(r, j), so, acc);
+          }
+          for (int t = 0; t < k; ++t) {
+            tile_t eb = Mfma<T>::zero(), acc = I::load(lo(r, t), so);
+            mma16<T>(eb, x, I::load(lo(k, t), so));
+            mma16<T>(acc, ua, eb);
+            I::store(lo(r, t), so, acc);
+          }
+          tile_t acc = Mfma<T>::zero();
+          mma16<T>(acc, ua, I::load(ed(k), so));
+          I::store(lo(r, k), so, acc);
+        }
+        if (w == k) put_diag(U, k);
+      }
+      extra(k);
+      __syncthreads();
+    }
+  }
+  __device__ __attribute__((always_inline)) inline void last_window(BSS_GLOBAL T* U) const {
+    const tile_t x = I::load(up(TT - 1, TT - 1), sa);
+    if (w < TT - 1)
+      finish(U, w, TT - 1, x);
+    else
+      put_diag(U, TT - 1);
+  }
+};
+
 // Waves per SIMD the registers are budgeted for (512 / this), from the workgroups that LDS
 // lets share a CU; every variant but n = 96 fits without spilling its strips.
 template <typename T, int NB>
@@ -313,8 +443,8 @@ __global__ void __launch_bounds__(4 * NB)
   // solve, or (LATE, where those registers spill) B in two halves before the solve and A
   // after it
   constexpr bool LATE = TT >= 6;
-  // W has tiles of its own in LDS up to n = 32; above that it takes C's place
-  constexpr bool OWN_W = TT <= 2;
+  // W has tiles of its own in LDS up to n = 48; above that it takes C's place
+  constexpr bool OWN_W = TT <= 3;
   typedef Img<T> I;
   typedef typename I::tile_t tile_t;
   // a lane's four elements of a tile in the input: vectors of 16 bytes
@@ -332,8 +462,6 @@ __global__ void __launch_bounds__(4 * NB)
   __shared__ __attribute__((aligned(16))) T Is[TS];            // the identity
   __shared__ int fail;
   auto up = [&](int r, int c) -> T* { return As + (c * (c + 1) / 2 + r) * TS; };
-  auto lo = [&](int i, int t) -> T* { return Ls + (i * (i - 1) / 2 + t) * TS; };
-  auto ed = [&](int k) -> T* { return Es + (k & 1) * TS; };
   auto ct = [&](int t, int c) -> T* { return Rs + (c * TT + t) * TS; };
   auto wt = [&](int t, int c) -> T* { return (OWN_W ? Vs : Rs) + (c * TT + t) * TS; };
 
@@ -350,12 +478,12 @@ __global__ void __launch_bounds__(4 * NB)
   const auto W = gptr((T*)S.W);
   const int w = wave_id();
   const int l = lane_id(), lr = l & 15, lk = l >> 4;
-  const int so = I::own_slot(), sa = I::a_slot(), ss = I::st_slot();
+  const int so = I::own_slot(), sa = I::a_slot();
+  const TileInverse<T, NB> inv{As, Ls, Es, Is, &fail, w, so, sa};
   // this lane's elements of a tile in global memory: its first vector (the second is
-  // DIV rows further), and of the lane order of the HBM stores
+  // DIV rows further)
   constexpr int DIV = sizeof(T) == 4 ? IV : 8;
   const int lcol = lr * NB + I::row(lk, 0);
-  const int scol = (l >> 2) * NB + I::VEC * (l & 3);
 
   struct raw_t {
     inv_t p[IP];
@@ -371,12 +499,6 @@ __global__ void __launch_bounds__(4 * NB)
 #pragma unroll
     for (int v = 0; v < 4; ++v) t[v] = (T)r.p[v / IV][v % IV];
     return t;
-  };
-  // a tile in LDS to HBM, times sg
-  auto put_img = [&](BSS_GLOBAL T* g, const T* tile, T f) {
-#pragma unroll
-    for (int h = 0; h < I::PLANES; ++h)
-      *gat<outv_t>(g + 8 * h, scol) = f * *(const outv_t*)(tile + 128 * h + I::VEC * ss);
   };
   // This wave's upper tiles (a, b) of a symmetric block: n = 0 is its diagonal tile, the
   // others go round.  The last ones may repeat a tile (in = false): a conditional load
@@ -460,9 +582,10 @@ __global__ void __launch_bounds__(4 * NB)
   auto store_w = [&](long long blk, T f) {
 #pragma unroll
     for (int t = 0; t < TT; ++t) I::store(wt(t, w), so, Ws[t]);
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-      put_img(W + blk * NN + 16 * w * NB + 16 * t, wt(t, w), f);
+    if (f > T(0))
+      put_tiles<T, NB, TT>(W + blk * NN + 16 * w * NB, wt(0, w));
+    else
+      put_tiles<T, NB, TT, true>(W + blk * NN + 16 * w * NB, wt(0, w));
   };
   auto s_left = [&]() {
 #pragma unroll
@@ -501,109 +624,37 @@ __global__ void __launch_bounds__(4 * NB)
       }
     }
 
-    // Windows k = -1 .. TT-1, one barrier each.  In window k < TT-1 wave k+1 updates diagonal tile
-    // k+1 with row k and factors it.  The other waves use Uinv_kk, published by window
-    // k-1: row i > k takes A(i, j) -= U_ki^T U_kj and E(i, t) -= U_ki^T E_kt, one row a
-    // wave, and the waves left over finish Uinv(t, k).  Every wave forms the tiles of row
-    // k that it needs itself (U_kj = Uinv_kk^T A_kj), so that row k is never rewritten and
-    // one barrier per diagonal tile is enough.  The rest of the windows goes to the
-    // previous block's Z' and S_L.
-    // Uinv(u, k) = (Uinv_kk^T E(k, u))^T, to LDS and HBM
-    auto finish = [&](int u, int k, const tile_t& x) {
-      tile_t e = Mfma<T>::zero();
-      mma16<T>(e, x, I::load(lo(k, u), so));
-      const auto g = U + blk * NN + 16 * k * NB + 16 * u;
-      const int olr = opaque_v(lr), olk = opaque_v(lk);
+    inv.windows(U + blk * NN, [&](int k) {
+      if (!late || TT == 1) return;
+      // The previous block's Z' and S_L, in windows in which the wave holds no diagonal
+      // tile.  Up to n = 48: all of it in windows -1 and 0.  Above: half of Z' in window
+      // -1 and half in window 0, what a wave missed in window 1; then W's tiles to LDS
+      // over C's, and S_L in window TT-1.
+      constexpr int H = OWN_W ? TT : TT / 2;
+      const bool first = (k == -1 && w != 0) || (k == (OWN_W ? 0 : 1) && w == 0);
+      const bool second = !OWN_W && ((k == 0 && w != 1) || (k == 1 && w == 1));
+      if (first) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        up(u, k)[I::off(olr, I::row(olk, v))] = e[v];
-        *gat<T>(g + (I::row(0, v)) * NB, I::row(olk, 0) * NB + olr) = e[v];
-      }
-    };
-    auto put_diag = [&](int k) {
-      put_img(U + blk * NN + 16 * k * NB + 16 * k, up(k, k), T(1));
-    };
-#pragma unroll 1
-    for (int k = -1; k < TT - 1; ++k) {
-      if (w == k + 1) {
-        if (k >= 0) {
-          const tile_t x = I::load(up(k, k), sa);
-          tile_t ub = Mfma<T>::zero(), acc = I::load(up(w, w), so);
-          mma16<T>(ub, x, I::load(up(k, w), so));
-          if constexpr (sizeof(T) == 4) {
-            mma16<T>(acc, -ub, ub);
-          } else {
-            tile_t ua = Mfma<T>::zero();
-            mma16<T>(ua, x, I::load(up(k, w), sa));
-            mma16<T>(acc, -ua, ub);
-          }
-          I::store(up(w, w), so, acc);
+        for (int a = 0; a < H; ++a) {
+          Zn[a] = z_tile(a);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        if (!diag_img<T>(up(w, w), up(w, w), ed(w), Is) && l == 0) fail = 1;
-      } else if (k >= 0) {
-        const tile_t x = I::load(up(k, k), sa);
-        const int u = w - (w > k + 1 ? 1 : 0);
-        if (u < k) {
-          finish(u, k, x);
-        } else {
-          const int r = u + 1;  // row r > k
-          tile_t ua = Mfma<T>::zero();
-          mma16<T>(ua, x, I::load(up(k, r), sa));
-          ua = -ua;
-          for (int j = (r == k + 1 ? r + 1 : r); j < TT; ++j) {
-            tile_t ub = Mfma<T>::zero(), acc = I::load(up(r, j), so);
-            mma16<T>(ub, x, I::load(up(k, j), so));
-            mma16<T>(acc, ua, ub);
-            I::store(up(r, j), so, acc);
-          }
-          for (int t = 0; t < k; ++t) {
-            tile_t eb = Mfma<T>::zero(), acc = I::load(lo(r, t), so);
-            mma16<T>(eb, x, I::load(lo(k, t), so));
-            mma16<T>(acc, ua, eb);
-            I::store(lo(r, t), so, acc);
-          }
-          tile_t acc = Mfma<T>::zero();
-          mma16<T>(acc, ua, I::load(ed(k), so));
-          I::store(lo(r, k), so, acc);
-        }
-        if (w == k) put_diag(k);
+        if (OWN_W) s_left();
       }
-      if (late && TT > 1) {
-        // Z': half of its tiles in window -1 and half in window 0, a wave busy with a
-        // diagonal tile there in window 1 (up to three tiles: all in windows -1, 0)
-        constexpr int H = TT >= 4 ? TT / 2 : TT;
-        const bool first = (k == -1 && w != 0) || (k == (TT >= 4 ? 1 : 0) && w == 0);
-        const bool second = TT >= 4 && ((k == 0 && w != 1) || (k == 1 && w == 1));
-        if (first) {
+      if (second) {
 #pragma unroll
-          for (int a = 0; a < H; ++a) {
-            Zn[a] = z_tile(a);
-            __builtin_amdgcn_sched_barrier(0);
-          }
+        for (int a = H; a < TT; ++a) {
+          Zn[a] = z_tile(a);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        if (second) {
-#pragma unroll
-          for (int a = H; a < TT; ++a) {
-            Zn[a] = z_tile(a);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-        if (!OWN_W && k == TT - 2) store_w(blk - 1, -sg);
       }
-      __syncthreads();
-    }
-    // Window TT-1
+      if (!OWN_W && k == TT - 2) store_w(blk - 1, -sg);
+    });
     raw_t br[LATE ? 1 : TT];  // the last block of the last chain has no coupling
     if (!LATE && hasC) load_b(br, blk, 0, TT);
-    {
-      const tile_t x = I::load(up(TT - 1, TT - 1), sa);
-      if (w < TT - 1)
-        finish(w, TT - 1, x);
-      else
-        put_diag(TT - 1);
-      if (late && TT > 1) s_left();
-      __syncthreads();
-    }
+    inv.last_window(U + blk * NN);
+    if (late && !OWN_W) s_left();
+    __syncthreads();
     if (threadIdx.x == 0 && fail) {
       fail_i = min(fail_i, i);
       fail = 0;
@@ -678,8 +729,7 @@ __global__ void __launch_bounds__(4 * NB)
     if (hasC) {
 #pragma unroll
       for (int t = 0; t < TT; ++t) I::store(ct(t, w), so, Cs[t]);
-#pragma unroll
-      for (int t = 0; t < TT; ++t) put_img(C + blk * NN + 16 * w * NB + 16 * t, ct(t, w), T(1));
+      put_tiles<T, NB, TT>(C + blk * NN + 16 * w * NB, ct(0, w));
     }
     if (OWN_W && hasL) store_w(blk, sg);
     if constexpr (FWD) {
@@ -760,6 +810,7 @@ __global__ void __launch_bounds__(4 * NB)
       }
       __syncthreads();  // A_{i+1} in LDS
     }
+    if (TT > 1) forget(Zn);  // written in the next block's windows
     sg = -sg;
   }
   if (hasL) {

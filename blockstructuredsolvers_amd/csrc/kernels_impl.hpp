@@ -3,8 +3,7 @@
 #pragma once
 
 #include "launch.hpp"
-#include "chain_factor_staged.hpp"
-#include "chain_factor_strip.hpp"
+#include "chain_factor_halves.hpp"
 #include "level_kernels.hpp"
 
 namespace bss {
@@ -25,10 +24,9 @@ static hipError_t factor_strip(const FactorLevelArgs& a, int nchains, hipStream_
 }
 
 // FP64 factors at n = 128 (no pivot monitor: only FP32 levels are monitored)
-static inline hipError_t factor_staged128(const FactorLevelArgs& a, int nchains, hipStream_t s) {
+static inline hipError_t factor_halves128(const FactorLevelArgs& a, int nchains, hipStream_t s) {
   if (a.fwd || a.pivmin) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((chain_factor_staged_kernel<double, double, 128, 8>), dim3(nchains),
-                     dim3(512), 0, s, a);
+  hipLaunchKernelGGL((chain_factor_halves_kernel<double, 128>), dim3(nchains), dim3(512), 0, s, a);
   return hipGetLastError();
 }
 
@@ -45,7 +43,7 @@ hipError_t launch_factor(int nb, const FactorLevelArgs& a, int nchains, hipStrea
       if constexpr (sizeof(T) == 4)
         return factor_strip<Tin, T, 128>(a, nchains, s);
       else
-        return factor_staged128(a, nchains, s);
+        return factor_halves128(a, nchains, s);
     default: return hipErrorInvalidValue;
   }
 }
