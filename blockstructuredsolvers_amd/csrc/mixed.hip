@@ -9,22 +9,16 @@
 #include "common.hpp"
 #include "mixed.hpp"
 #include "pinned_pool.hpp"
+#include "residual_column.hpp"
 
 namespace bss {
 namespace {
 
 thread_local std::string g_mixed_err;
-// per workgroup partials: [0,16) max|r_j|, [16,32) max|x_j|, [32,48) max|d_j|,
-// [48] max row sum of |M| (when requested)
-constexpr int kParts = 64;
-constexpr int kMnormSlot = 48;
-
 size_t al(size_t b) { return (b + 255) & ~size_t(255); }
 
-// NaN-propagating max (fmax would drop a NaN residual and report convergence)
-__device__ inline double nmax(double a, double b) { return (b > a || b != b) ? b : a; }
-
-// Residual pass over one work item (a block range [b0, b1) of one system):
+// Residual pass over one work item (a block range [b0, b1) of one system), several
+// right-hand sides:
 //   x_new = x_old + dx (FP64; written for the workgroup's own blocks),
 //   r = d - (B_{i-1}^T x_{i-1} + A_i x_i + B_i x_{i+1}) in FP64 on MFMA, stored as FP32
 //   for the next correction solve, plus per-column max |r|, |x|, |d|.
@@ -35,98 +29,17 @@ __device__ inline double nmax(double a, double b) { return (b > a || b != b) ? b
 // Every coupling block is read from HBM once: at block row i, B_i serves both
 // B_i x_{i+1} (row i) and B_i^T x_i (row i+1, carried to the next iteration in
 // registers); the second read of B_i follows the first immediately and hits L2.
-// V1 (one right-hand side): the products are FP64 FMAs on the same operand registers
-// instead of MFMA.  A 16x16x4 FP64 MFMA issues every 64 cycles on this GPU, the same
-// FLOP rate as the vector FMAs, but with one column it would compute 16 columns to keep
-// one; each lane then sums its 16 k-slots and the four lanes of a row combine.
-// TS (V1 up to n = 64, no ||M|| pass): B_i^T x_i is not read again from L2 as a
-// transposed operand; the products B_i[r][k] x_i[r] of the registers that serve B_i
-// x_{i+1} go to an LDS tile, and the next row sums its columns.
-// RQ (V1 from n = 96 on, where that tile would not fit in LDS, and at n = 64 with the
-// ||M|| pass): the same products are summed over the 16 rows of each wave in registers
-// (red16) and only the per-wave sums go to LDS, n values per wave; the next row adds the
-// waves' sums.  The ||M|| pass sums |B_i| the same way.  The transposed re-read of B_i
-// it replaces ran this kernel at 3.7 TB/s at n = 128 (its strided 32-byte reads),
-// against 5.6 without it; at n = 64 the ||M|| residual went from 3.56 to 3.42 ms for
-// 32 systems, while without ||M|| the LDS tile stays as fast (3.29 against 3.32 ms).
-template <int KC>
-struct Red16 {
-  // halving steps (masks 8, 4, ..) while the slot count stays even; the rest exchange
-  // whole values
-  static constexpr int halvings() {
-    int v = KC, h = 0;
-    while (h < 4 && v % 2 == 0) {
-      v /= 2;
-      ++h;
-    }
-    return h;
-  }
-  static constexpr int H = halvings();
-  static constexpr int CNT = KC >> H;  // sums each lane holds at the end
-};
-
-// Sums KC values of every lane over the 16 lanes of its row group (lanes l ^ 1, 2, 4,
-// 8).  Halving step with mask m: the lane whose mask bit is clear keeps the first half of
-// its slots, the other the second half, and each adds the partner's copy of the half it
-// keeps; then whole exchanges for the masks left.  On return v[0 .. CNT) of lane lr are
-// the sums of local slots red16_first(lr) .. + CNT (the same in lanes that differ only in
-// the exchanged mask bits).
-template <int KC>
-__device__ inline void red16(double (&v)[KC], int lr) {
-  constexpr int H = Red16<KC>::H;
-  int V = KC;
-#pragma unroll
-  for (int i = 0; i < H; ++i) {
-    const int m = 8 >> i;
-    const bool up = (lr & m) != 0;
-    const int half = V / 2;
-#pragma unroll
-    for (int j = 0; j < KC / 2; ++j) {
-      if (j < half) {
-        const double send = up ? v[j] : v[half + j];
-        const double recv = __shfl_xor(send, m);
-        v[j] = (up ? v[half + j] : v[j]) + recv;
-      }
-    }
-    V = half;
-  }
-#pragma unroll
-  for (int i = H; i < 4; ++i) {
-    const int m = 8 >> i;
-#pragma unroll
-    for (int j = 0; j < Red16<KC>::CNT; ++j) v[j] += __shfl_xor(v[j], m);
-  }
-}
-template <int KC>
-__device__ inline int red16_first(int lr) {
-  int f = 0, V = KC;
-#pragma unroll
-  for (int i = 0; i < Red16<KC>::H; ++i) {
-    V /= 2;
-    if (lr & (8 >> i)) f += V;
-  }
-  return f;
-}
-
-// MN: the ||M|| pass may run (taken from mnorm_arg for several columns; one-column
-// kernels are launched with MN equal to it, which keeps branches out of their k loop).
-template <int NB, bool V1, bool TS, bool MN>
+// (One right-hand side: residual_column_kernel.)
+template <int NB>
 __global__ void __launch_bounds__(4 * NB)
     residual_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
                     double* __restrict__ part, int nrhs, int xo_k, int dx_k, int xn_k, int ro_k,
-                    int mnorm_arg) {
-  static_assert(!TS || (V1 && NB <= 64 && !MN), "transpose-sum path: one column, n <= 64");
+                    int mnorm) {
   constexpr int TT = NB / 16, NT = 64 * TT, LDV = NB + 2, KQ = NB / 4;
   constexpr long long NN = (long long)NB * NB;
   typedef Mfma<double>::acc_t acc_t;
   __shared__ double X[3][16 * LDV];
   __shared__ double red[4][4 * TT][16];
-  constexpr int LDP = NB + 1;
-  __shared__ double P[TS ? NB * LDP : 1];  // TS: B_i[r][k] x_i[r] at P[r * LDP + k]
-  constexpr bool RQ = V1 && !TS && NB >= 64;
-  // RQ: per-wave sums over rows r of B_i[r][k] x_i[r] (Q[0]) and |B_i[r][k]| (Q[1])
-  __shared__ double Q[RQ ? 2 : 1][RQ ? TT * NB : 1];
-  const int mnorm = !MN ? 0 : V1 ? 1 : mnorm_arg;
   const ResItem it = items[blockIdx.x];
   const ResSys& S = systems[it.sys];
   const int N = S.N;
@@ -136,8 +49,8 @@ __global__ void __launch_bounds__(4 * NB)
   const auto As = gptr((const double*)S.A);
   const auto Bs = gptr((const double*)S.B);
   const auto ds = gptr((const double*)S.d);
-  const auto xo = gptr((const double*)(xo_k >= 0 ? S.x[xo_k] : nullptr));
-  const auto dxs = gptr((const float*)(dx_k >= 0 ? S.v[dx_k] : nullptr));
+  const auto xo = gptr((const double*)S.x[xo_k]);
+  const auto dxs = gptr((const float*)S.v[dx_k]);
   const auto xn = gptr(S.x[xn_k]);
   const auto ro = gptr(S.v[ro_k]);
   for (int e = tid; e < 3 * 16 * LDV; e += NT) (&X[0][0])[e] = 0.0;
@@ -183,12 +96,8 @@ __global__ void __launch_bounds__(4 * NB)
   // k index of operand slot q: 4 consecutive k per lane (contiguous loads along k)
   auto kof = [&](int q) { return (q >> 2) * 16 + 4 * lk + (q & 3); };
 
-  // sum over the four lanes (lk) that share row 16w + lr
-  auto row_sum = [&](double v) { return row4_sum(v); };
-  // carry: B_{i-1}^T x_{i-1} for the current row (and its |.| row sums for ||M||_inf);
-  // V1 keeps it as one value per lane (row 16w + lr)
+  // carry: B_{i-1}^T x_{i-1} for the current row (and its |.| row sums for ||M||_inf)
   acc_t carry = Mfma<double>::zero();
-  [[maybe_unused]] double carry1 = 0.0;
   double rs_carry = 0.0;
   __syncthreads();  // window zeroed
   {
@@ -204,262 +113,96 @@ __global__ void __launch_bounds__(4 * NB)
     __syncthreads();
     if (has) {
       const double* Xm = X[(((b0 - 1) % 3) + 3) % 3];
-      if constexpr (V1) {
-        double t = 0.0;
-#pragma unroll
-        for (int q = 0; q < KQ; ++q) t = fma(aBt[q], Xm[kof(q)], t);
-        carry1 = row_sum(t);
-      }
 #pragma unroll
       for (int q = 0; q < KQ; ++q) {
-        if constexpr (!V1) carry = Mfma<double>::mma(aBt[q], Xm[lr * LDV + kof(q)], carry);
+        carry = Mfma<double>::mma(aBt[q], Xm[lr * LDV + kof(q)], carry);
         if (mnorm) rs_carry += fabs(aBt[q]);
-      }
-      if constexpr (RQ) {
-        if (mnorm) rs_carry = row4_sum(rs_carry);  // RQ keeps whole row sums
       }
     }
   }
 
-  // the k range in NCH chunks of KC operand slots (two chunks from n = 64 on with MFMA),
-  // which bounds the operand registers and measured faster at n = 64; V1 up to n = 64
-  // holds fewer registers and takes one chunk (at n = 128 one chunk would spill)
-  constexpr int KC = ((V1 && NB <= 64) || KQ <= 8 || KQ % 8 != 0) ? KQ : KQ / 2;
+  // the k range in NCH chunks of KC operand slots (two chunks from n = 64 on), which
+  // bounds the operand registers and measured faster at n = 64
+  constexpr int KC = (KQ <= 8 || KQ % 8 != 0) ? KQ : KQ / 2;
   constexpr int NCH = KQ / KC;
   static_assert(KC * NCH == KQ && KC % 4 == 0, "operand chunks");
-  // PF: A of the next block row is loaded one row ahead, after this row's other loads,
-  // so that it is still in flight while this row waits for them (V1 at n <= 64, where
-  // the registers allow it; the last row of an item re-reads its own block from L2)
-  constexpr bool PF = V1 && NB <= 64;
-  double pA[KQ];
-  if constexpr (PF) {
-#pragma unroll
-    for (int q = 0; q < KQ; ++q) pA[q] = As[b0 * NN + (long long)kof(q) * NB + 16 * w + lr];
-  }
-  // RQ runs in two chunks from n = 96 on (one at n = 64).  EO (explicit order): the
-  // second chunk's loads are issued before the first chunk's work; left to itself the scheduler issues them after it,
-  // and a work-group (one per CU at n = 128) then has half a block row in flight.
-  // At n = 96 the registers this takes cost the second work-group per CU, and the
-  // scheduler's own order measured faster.
-  constexpr bool EO = RQ && NB >= 128;
-  static_assert(!EO || NCH == 2, "explicit order: two chunks");
   for (int blk = b0; blk < b1; ++blk) {
     // operands of this block row, issued first; B_blk twice (row blk, and transposed
-    // for row blk + 1 when that row is ours) unless TS or RQ carries B^T x
+    // for row blk + 1 when that row is ours)
     const bool next = blk + 1 < N;
     const bool carry_on = next && blk + 1 < b1;
     double xs[SE];
     stage_load(blk + 1, xs);
     double aA[KC], aB[KC], aBn[KC];
-    double cA[EO ? KC : 1], cB[EO ? KC : 1];  // EO: chunk 0
     // B_blk exists only below the last block; otherwise its loads read A_blk (always
     // there) and are zeroed, so no load is conditional
     const auto Bb = next ? Bs + blk * NN : As + blk * NN;
-    auto load_ops = [&](int ch, double(&uA)[KC], double(&uB)[KC]) {
+    auto load_chunk = [&](int ch) {
 #pragma unroll
       for (int qq = 0; qq < KC; ++qq) {
         const int k = kof(ch * KC + qq);
-        if constexpr (PF) uA[qq] = pA[ch * KC + qq];
-        else uA[qq] = As[blk * NN + (long long)k * NB + 16 * w + lr];
+        aA[qq] = As[blk * NN + (long long)k * NB + 16 * w + lr];
         const double b = Bb[(long long)k * NB + 16 * w + lr];
-        uB[qq] = next ? b : 0.0;
+        aB[qq] = next ? b : 0.0;
       }
-    };
-    auto load_chunk = [&](int ch) {
-      load_ops(ch, aA, aB);
-      if constexpr (!TS && !RQ) {
 #pragma unroll
-        for (int qq = 0; qq < KC; ++qq) {
-          const double b = Bb[(long long)(16 * w + lr) * NB + kof(ch * KC + qq)];
-          aBn[qq] = carry_on ? b : 0.0;
-        }
+      for (int qq = 0; qq < KC; ++qq) {
+        const double b = Bb[(long long)(16 * w + lr) * NB + kof(ch * KC + qq)];
+        aBn[qq] = carry_on ? b : 0.0;
       }
     };
     // d_blk, like x, ahead of the operands
     acc_t acc;
-    [[maybe_unused]] double d1 = 0.0;
-    if constexpr (V1) {
-      d1 = ds[(long long)blk * ND + 16 * w + lr];
-    } else {
-      const int dc = lr < nrhs ? lr : 0;
+    const int dc = lr < nrhs ? lr : 0;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * w + Mfma<double>::row(lk, v);
-        const double x = ds[(long long)blk * ND + dc * NB + row];
-        acc[v] = (lr < nrhs) ? x : 0.0;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * w + Mfma<double>::row(lk, v);
+      const double x = ds[(long long)blk * ND + dc * NB + row];
+      acc[v] = (lr < nrhs) ? x : 0.0;
     }
-    if constexpr (!EO) load_chunk(0);
-    else load_ops(0, cA, cB);
-    if constexpr (PF) {
-      const int j = blk + 1 < b1 ? blk + 1 : blk;
+    load_chunk(0);
 #pragma unroll
-      for (int q = 0; q < KQ; ++q) pA[q] = As[j * NN + (long long)kof(q) * NB + 16 * w + lr];
-    }
-    if constexpr (V1) {
-      dmax = nmax(dmax, fabs(d1));
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) dmax = nmax(dmax, fabs(acc[v]));
-    }
+    for (int v = 0; v < 4; ++v) dmax = nmax(dmax, fabs(acc[v]));
     __syncthreads();  // previous block's window reads are done
-    if constexpr (TS) {
-      // this row's carry: column 16w + lr of the previous row's product tile (written
-      // after the previous row's second barrier, rewritten only after this row's)
-      // (the four lanes of a row each sum NB / 4 of the tile's rows)
-      if (blk > b0) {
-        double t = 0.0;
-#pragma unroll
-        for (int r = 0; r < NB / 4; ++r) t += P[((NB / 4) * lk + r) * LDP + 16 * w + lr];
-        carry1 = row_sum(t);
-      }
-    }
-    if constexpr (RQ) {
-      // this row's carry (and |B| row sum): the previous row's per-wave sums (written
-      // after the previous row's second barrier, rewritten only after this row's)
-      if (blk > b0) {
-        double t = 0.0, u = 0.0;
-#pragma unroll
-        for (int v = 0; v < TT; ++v) {
-          t += Q[0][v * NB + 16 * w + lr];
-          if (mnorm) u += Q[1][v * NB + 16 * w + lr];
-        }
-        carry1 = t;
-        if (mnorm) rs_carry = u;
-      }
-    }
     stage_store(blk + 1, xs);
     __syncthreads();
     const double* X0 = X[blk % 3];
     const double* Xp = X[(blk + 1) % 3];
-    if constexpr (V1) {
-      xmax = nmax(xmax, fabs(X0[16 * w + lr]));
-    } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        xmax = nmax(xmax, fabs(X0[lr * LDV + 16 * w + Mfma<double>::row(lk, v)]));
-    }
-    {
-      if constexpr (!V1) {
+    for (int v = 0; v < 4; ++v)
+      xmax = nmax(xmax, fabs(X0[lr * LDV + 16 * w + Mfma<double>::row(lk, v)]));
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[v] -= carry[v];
-      }
-      acc_t cn = Mfma<double>::zero();
-      // V1 partial sums: A x and B x in two chains, B^T x (the next row's carry)
-      [[maybe_unused]] double sa = 0.0, sb = 0.0, sn = 0.0;
-      double rs = RQ ? 0.0 : rs_carry, rsn = 0.0;
-      // RQ: the next row's carry, B[r][k] x[r] summed over the wave's 16 rows (and
-      // |B[r][k]| for ||M||), to Q[.][w NB + k], for slots q0 .. q0 + G of chunk ch as
-      // their FMAs end (a whole chunk at once spills at n = 128).  No branch (a branch
-      // splits the unrolled loop and its loads then spill): every lane stores, the lanes
-      // that share a sum hold the same bits (its adds are commutative); rows without a
-      // next row in this item store sums nobody reads.
-      constexpr int G = KC % 8 == 0 ? 8 : 4;
-      auto rq_sums = [&](int ch, int q0, const double(&uB)[KC]) {
-        constexpr int CNT = Red16<G>::CNT;
-        const int f = red16_first<G>(lr);
-        const double xr = X0[16 * w + lr];
-        double t[G];
+    for (int v = 0; v < 4; ++v) acc[v] -= carry[v];
+    acc_t cn = Mfma<double>::zero();
+    double rs = rs_carry, rsn = 0.0;
 #pragma unroll
-        for (int j = 0; j < G; ++j) t[j] = uB[q0 + j] * xr;
-        red16<G>(t, lr);
+    for (int ch = 0; ch < NCH; ++ch) {
+      if (ch > 0) load_chunk(ch);
 #pragma unroll
-        for (int c = 0; c < CNT; ++c) Q[0][w * NB + kof(ch * KC + q0 + f + c)] = t[c];
+      for (int qq = 0; qq < KC; ++qq) {
+        const int k = kof(ch * KC + qq);
+        acc = Mfma<double>::mma(-aA[qq], X0[lr * LDV + k], acc);
+        acc = Mfma<double>::mma(-aB[qq], Xp[lr * LDV + k], acc);
+        cn = Mfma<double>::mma(aBn[qq], X0[lr * LDV + k], cn);
         if (mnorm) {
-#pragma unroll
-          for (int j = 0; j < G; ++j) t[j] = fabs(uB[q0 + j]);
-          red16<G>(t, lr);
-#pragma unroll
-          for (int c = 0; c < CNT; ++c) Q[1][w * NB + kof(ch * KC + q0 + f + c)] = t[c];
+          rs += fabs(aA[qq]) + fabs(aB[qq]);
+          rsn += fabs(aBn[qq]);
         }
-      };
-      if constexpr (EO) {
-        auto chunk_work = [&](int ch, const double(&uA)[KC], const double(&uB)[KC]) {
-#pragma unroll
-          for (int qq = 0; qq < KC; ++qq) {
-            const int k = kof(ch * KC + qq);
-            sa = fma(uA[qq], X0[k], sa);
-            sb = fma(uB[qq], Xp[k], sb);
-            if (mnorm) rs += fabs(uA[qq]) + fabs(uB[qq]);
-            if (qq % G == G - 1) rq_sums(ch, qq + 1 - G, uB);
-          }
-        };
-        // chunk 1's loads, then chunk 0's work, kept in that order by the barrier
-        double nA[KC], nB[KC];
-        load_ops(1, nA, nB);
-        __builtin_amdgcn_sched_barrier(0);
-        chunk_work(0, cA, cB);
-        chunk_work(1, nA, nB);
-      } else {
-#pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) {
-          if (ch > 0) load_chunk(ch);
-#pragma unroll
-          for (int qq = 0; qq < KC; ++qq) {
-            const int k = kof(ch * KC + qq);
-            if constexpr (V1) {
-              const double x0 = X0[k];
-              sa = fma(aA[qq], x0, sa);
-              sb = fma(aB[qq], Xp[k], sb);
-              if constexpr (!TS && !RQ) sn = fma(aBn[qq], x0, sn);
-            } else {
-              acc = Mfma<double>::mma(-aA[qq], X0[lr * LDV + k], acc);
-              acc = Mfma<double>::mma(-aB[qq], Xp[lr * LDV + k], acc);
-              cn = Mfma<double>::mma(aBn[qq], X0[lr * LDV + k], cn);
-            }
-            if (mnorm) {
-              rs += fabs(aA[qq]) + fabs(aB[qq]);
-              if constexpr (!RQ) rsn += fabs(aBn[qq]);
-            }
-            if constexpr (RQ) {
-              if (qq % G == G - 1) rq_sums(ch, qq + 1 - G, aB);
-            }
-          }
-        }
-      }
-      if constexpr (TS) {
-        d1 = d1 - carry1 - row_sum(sa + sb);
-        if (carry_on) {
-          const double xr = X0[16 * w + lr];
-#pragma unroll
-          for (int q = 0; q < KQ; ++q) P[(16 * w + lr) * LDP + kof(q)] = aB[q] * xr;
-        }
-      } else if constexpr (V1 && RQ) {
-        d1 = d1 - carry1 - row_sum(sa + sb);  // the next carry comes through Q
-      } else if constexpr (V1) {
-        d1 = d1 - carry1 - row_sum(sa + sb);
-        carry1 = row_sum(sn);
-      } else {
-        carry = cn;
-      }
-      if constexpr (!RQ) rs_carry = rsn;
-      if (mnorm) {
-        // the four lanes sharing lr hold the four k-slices of row 16w + lr
-        rs = row4_sum(rs);
-        if constexpr (RQ) rs += rs_carry;  // the |B_{i-1}| column sum, already whole
-        mmax = nmax(mmax, rs);
       }
     }
-    if constexpr (V1) {
-      if (lk == 0) ro[(long long)blk * ND + 16 * w + lr] = (float)d1;
-      rmax = nmax(rmax, fabs(d1));
-    } else if (lr < nrhs) {
+    carry = cn;
+    rs_carry = rsn;
+    if (mnorm) {
+      // the four lanes sharing lr hold the four k-slices of row 16w + lr
+      mmax = nmax(mmax, row4_sum(rs));
+    }
+    if (lr < nrhs) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         ro[(long long)blk * ND + lr * NB + 16 * w + Mfma<double>::row(lk, v)] = (float)acc[v];
         rmax = nmax(rmax, fabs(acc[v]));
       }
     }
-  }
-  if constexpr (V1) {
-    // lanes hold rows of column 0: fold the wave into column slot 0
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      rmax = nmax(rmax, __shfl_xor(rmax, o));
-      xmax = nmax(xmax, __shfl_xor(xmax, o));
-      dmax = nmax(dmax, __shfl_xor(dmax, o));
-    }
-    if (lr != 0) rmax = xmax = dmax = 0.0;
   }
   red[0][4 * w + lk][lr] = rmax;
   red[1][4 * w + lk][lr] = xmax;
@@ -584,16 +327,14 @@ hipError_t launch_residual(const MixedState& m, bool init, int xo_k, int dx_k, i
     hipLaunchKernelGGL(init_pass_kernel, dim3(m.nitems), dim3(kInitThreads), 0, s, m.items,
                        m.sys_dev, m.part, NB, m.nrhs, xn_k, ro_k, m.init_skip);
   else if (m.nrhs == 1 && !want_mnorm)
-    hipLaunchKernelGGL((residual_kernel<NB, true, NB <= 64, false>), dim3(m.nitems),
-                       dim3(4 * NB), 0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k,
-                       ro_k, 0);
+    hipLaunchKernelGGL((residual_column_kernel<NB, false>), dim3(m.nitems), dim3(64 * kColWaves),
+                       0, s, m.items, m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
   else if (m.nrhs == 1)
-    hipLaunchKernelGGL((residual_kernel<NB, true, false, true>), dim3(m.nitems), dim3(4 * NB),
-                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k, 1);
+    hipLaunchKernelGGL((residual_column_kernel<NB, true>), dim3(m.nitems), dim3(64 * kColWaves),
+                       0, s, m.items, m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
   else
-    hipLaunchKernelGGL((residual_kernel<NB, false, false, true>), dim3(m.nitems), dim3(4 * NB),
-                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k,
-                       want_mnorm);
+    hipLaunchKernelGGL((residual_kernel<NB>), dim3(m.nitems), dim3(4 * NB), 0, s, m.items,
+                       m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k, want_mnorm);
   return hipGetLastError();
 }
 
