@@ -10,217 +10,13 @@
 #include "mixed.hpp"
 #include "pinned_pool.hpp"
 #include "residual_column.hpp"
+#include "residual_tiles.hpp"
 
 namespace bss {
 namespace {
 
 thread_local std::string g_mixed_err;
 size_t al(size_t b) { return (b + 255) & ~size_t(255); }
-
-// Residual pass over one work item (a block range [b0, b1) of one system), several
-// right-hand sides:
-//   x_new = x_old + dx (FP64; written for the workgroup's own blocks),
-//   r = d - (B_{i-1}^T x_{i-1} + A_i x_i + B_i x_{i+1}) in FP64 on MFMA, stored as FP32
-//   for the next correction solve, plus per-column max |r|, |x|, |d|.
-// With `mnorm`, the row sums of |M| are accumulated from the operand values the
-// products already hold, so ||M||_inf costs no extra pass over A and B.
-// One wave per 16-row tile; a rolling three-block window of x_new lives in LDS and
-// each block's A/B operands are issued before the window update to hide HBM latency.
-// Every coupling block is read from HBM once: at block row i, B_i serves both
-// B_i x_{i+1} (row i) and B_i^T x_i (row i+1, carried to the next iteration in
-// registers); the second read of B_i follows the first immediately and hits L2.
-// (One right-hand side: residual_column_kernel.)
-template <int NB>
-__global__ void __launch_bounds__(4 * NB)
-    residual_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
-                    double* __restrict__ part, int nrhs, int xo_k, int dx_k, int xn_k, int ro_k,
-                    int mnorm) {
-  constexpr int TT = NB / 16, NT = 64 * TT, LDV = NB + 2, KQ = NB / 4;
-  constexpr long long NN = (long long)NB * NB;
-  typedef Mfma<double>::acc_t acc_t;
-  __shared__ double X[3][16 * LDV];
-  __shared__ double red[4][4 * TT][16];
-  const ResItem it = items[blockIdx.x];
-  const ResSys& S = systems[it.sys];
-  const int N = S.N;
-  const int tid = threadIdx.x;
-  const int w = wave_id(), l = lane_id(), lr = l & 15, lk = l >> 4;
-  const long long ND = (long long)NB * nrhs;
-  const auto As = gptr((const double*)S.A);
-  const auto Bs = gptr((const double*)S.B);
-  const auto ds = gptr((const double*)S.d);
-  const auto xo = gptr((const double*)S.x[xo_k]);
-  const auto dxs = gptr((const float*)S.v[dx_k]);
-  const auto xn = gptr(S.x[xn_k]);
-  const auto ro = gptr(S.v[ro_k]);
-  for (int e = tid; e < 3 * 16 * LDV; e += NT) (&X[0][0])[e] = 0.0;
-  double rmax = 0.0, xmax = 0.0, dmax = 0.0, mmax = 0.0;
-  const int b0 = it.b0, b1 = it.b1;
-
-  // x_new of block j (zero outside the system), elements e = tid + u*NT: loaded into
-  // registers by stage_load, then written to its window slot (and, for the
-  // workgroup's own blocks, to xnew) by stage_store.  The wait counters are in order,
-  // so the x loads are issued before the block's operand loads, and the wait for them
-  // leaves the operands in flight; every lane loads (clamped indices), as a predicated
-  // load would make every later wait conservative.  x_old and dx are always given
-  // (the first pass of a solve is init_pass_kernel).
-  constexpr int SE = (NB * 16 + NT - 1) / NT;  // up to 16 right-hand sides
-  auto stage_load = [&](int j, double (&v)[SE]) {
-    const bool inside = j >= 0 && j < N;
-    const long long jc = j < 0 ? 0 : (j >= N ? N - 1 : j);
-#pragma unroll
-    for (int u = 0; u < SE; ++u) {
-      const int e = tid + u * NT;
-      const long long o = jc * ND + (e < (int)ND ? e : 0);
-      const double x = xo[o] + (double)dxs[o];
-      v[u] = inside ? x : 0.0;
-    }
-  };
-  auto stage_store = [&](int j, const double (&v)[SE]) {
-    double* slot = X[((j % 3) + 3) % 3];
-    const bool own = j >= b0 && j < b1;
-#pragma unroll
-    for (int u = 0; u < SE; ++u) {
-      const int e = tid + u * NT;
-      if (e < (int)ND) {
-        slot[(e / NB) * LDV + (e % NB)] = v[u];
-        if (own) xn[(long long)j * ND + e] = v[u];
-      }
-    }
-  };
-  auto stage = [&](int j) {
-    double v[SE];
-    stage_load(j, v);
-    stage_store(j, v);
-  };
-  // k index of operand slot q: 4 consecutive k per lane (contiguous loads along k)
-  auto kof = [&](int q) { return (q >> 2) * 16 + 4 * lk + (q & 3); };
-
-  // carry: B_{i-1}^T x_{i-1} for the current row (and its |.| row sums for ||M||_inf)
-  acc_t carry = Mfma<double>::zero();
-  double rs_carry = 0.0;
-  __syncthreads();  // window zeroed
-  {
-    double aBt[KQ];
-    const bool has = b0 > 0;
-    if (has) {
-#pragma unroll
-      for (int q = 0; q < KQ; ++q)
-        aBt[q] = Bs[(b0 - 1) * NN + (long long)(16 * w + lr) * NB + kof(q)];
-    }
-    stage(b0 - 1);
-    stage(b0);
-    __syncthreads();
-    if (has) {
-      const double* Xm = X[(((b0 - 1) % 3) + 3) % 3];
-#pragma unroll
-      for (int q = 0; q < KQ; ++q) {
-        carry = Mfma<double>::mma(aBt[q], Xm[lr * LDV + kof(q)], carry);
-        if (mnorm) rs_carry += fabs(aBt[q]);
-      }
-    }
-  }
-
-  // the k range in NCH chunks of KC operand slots (two chunks from n = 64 on), which
-  // bounds the operand registers and measured faster at n = 64
-  constexpr int KC = (KQ <= 8 || KQ % 8 != 0) ? KQ : KQ / 2;
-  constexpr int NCH = KQ / KC;
-  static_assert(KC * NCH == KQ && KC % 4 == 0, "operand chunks");
-  for (int blk = b0; blk < b1; ++blk) {
-    // operands of this block row, issued first; B_blk twice (row blk, and transposed
-    // for row blk + 1 when that row is ours)
-    const bool next = blk + 1 < N;
-    const bool carry_on = next && blk + 1 < b1;
-    double xs[SE];
-    stage_load(blk + 1, xs);
-    double aA[KC], aB[KC], aBn[KC];
-    // B_blk exists only below the last block; otherwise its loads read A_blk (always
-    // there) and are zeroed, so no load is conditional
-    const auto Bb = next ? Bs + blk * NN : As + blk * NN;
-    auto load_chunk = [&](int ch) {
-#pragma unroll
-      for (int qq = 0; qq < KC; ++qq) {
-        const int k = kof(ch * KC + qq);
-        aA[qq] = As[blk * NN + (long long)k * NB + 16 * w + lr];
-        const double b = Bb[(long long)k * NB + 16 * w + lr];
-        aB[qq] = next ? b : 0.0;
-      }
-#pragma unroll
-      for (int qq = 0; qq < KC; ++qq) {
-        const double b = Bb[(long long)(16 * w + lr) * NB + kof(ch * KC + qq)];
-        aBn[qq] = carry_on ? b : 0.0;
-      }
-    };
-    // d_blk, like x, ahead of the operands
-    acc_t acc;
-    const int dc = lr < nrhs ? lr : 0;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = 16 * w + Mfma<double>::row(lk, v);
-      const double x = ds[(long long)blk * ND + dc * NB + row];
-      acc[v] = (lr < nrhs) ? x : 0.0;
-    }
-    load_chunk(0);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) dmax = nmax(dmax, fabs(acc[v]));
-    __syncthreads();  // previous block's window reads are done
-    stage_store(blk + 1, xs);
-    __syncthreads();
-    const double* X0 = X[blk % 3];
-    const double* Xp = X[(blk + 1) % 3];
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      xmax = nmax(xmax, fabs(X0[lr * LDV + 16 * w + Mfma<double>::row(lk, v)]));
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[v] -= carry[v];
-    acc_t cn = Mfma<double>::zero();
-    double rs = rs_carry, rsn = 0.0;
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-      if (ch > 0) load_chunk(ch);
-#pragma unroll
-      for (int qq = 0; qq < KC; ++qq) {
-        const int k = kof(ch * KC + qq);
-        acc = Mfma<double>::mma(-aA[qq], X0[lr * LDV + k], acc);
-        acc = Mfma<double>::mma(-aB[qq], Xp[lr * LDV + k], acc);
-        cn = Mfma<double>::mma(aBn[qq], X0[lr * LDV + k], cn);
-        if (mnorm) {
-          rs += fabs(aA[qq]) + fabs(aB[qq]);
-          rsn += fabs(aBn[qq]);
-        }
-      }
-    }
-    carry = cn;
-    rs_carry = rsn;
-    if (mnorm) {
-      // the four lanes sharing lr hold the four k-slices of row 16w + lr
-      mmax = nmax(mmax, row4_sum(rs));
-    }
-    if (lr < nrhs) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        ro[(long long)blk * ND + lr * NB + 16 * w + Mfma<double>::row(lk, v)] = (float)acc[v];
-        rmax = nmax(rmax, fabs(acc[v]));
-      }
-    }
-  }
-  red[0][4 * w + lk][lr] = rmax;
-  red[1][4 * w + lk][lr] = xmax;
-  red[2][4 * w + lk][lr] = dmax;
-  red[3][4 * w + lk][lr] = mmax;
-  __syncthreads();
-  if (tid < kParts) {
-    const int q = tid / 16, c = tid % 16;
-    double m = 0.0;
-    if (q < 3) {
-      for (int k = 0; k < 4 * TT; ++k) m = nmax(m, red[q][k][c]);
-    } else if (c == 0) {
-      for (int k = 0; k < 4 * TT; ++k)
-        for (int cc = 0; cc < 16; ++cc) m = nmax(m, red[3][k][cc]);
-    }
-    if (q < 3 || c == 0) part[(long long)blockIdx.x * kParts + (q < 3 ? tid : kMnormSlot)] = m;
-  }
-}
 
 // Combine the partial maxima: berr per (system, column).  `init` records ||d_j||;
 // `mnorm` first reduces ||M||_inf from the same pass.  One kRedThreads workgroup per
@@ -332,9 +128,12 @@ hipError_t launch_residual(const MixedState& m, bool init, int xo_k, int dx_k, i
   else if (m.nrhs == 1)
     hipLaunchKernelGGL((residual_column_kernel<NB, true>), dim3(m.nitems), dim3(64 * kColWaves),
                        0, s, m.items, m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
+  else if (!want_mnorm)
+    hipLaunchKernelGGL((residual_tiles_kernel<NB, false>), dim3(m.nitems), dim3(64 * kColWaves),
+                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
   else
-    hipLaunchKernelGGL((residual_kernel<NB>), dim3(m.nitems), dim3(4 * NB), 0, s, m.items,
-                       m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k, want_mnorm);
+    hipLaunchKernelGGL((residual_tiles_kernel<NB, true>), dim3(m.nitems), dim3(64 * kColWaves),
+                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
   return hipGetLastError();
 }
 

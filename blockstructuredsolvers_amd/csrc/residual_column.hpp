@@ -94,7 +94,8 @@ constexpr int kColWaves = 4;  // waves of a work-group: block rows of an item in
 // Eight waves a work-group at 128 registers spill; four at 168 give the same bytes in
 // flight.
 template <int NB, bool MN>
-__global__ void __launch_bounds__(64 * kColWaves) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(64 * kColWaves)
+    __attribute__((amdgpu_waves_per_eu(NB == 96 && MN ? 2 : 3)))  // (LDS: two work-groups a CU)
     residual_column_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
                            double* __restrict__ part, int xo_k, int dx_k, int xn_k, int ro_k) {
   typedef ColMap<NB> M;

@@ -12,6 +12,7 @@
  *           every block column-major with leading dimension n, blocks contiguous,
  *           A : n*n*N, B : n*n*(N-1), d : n*nrhs*N elements per system; a batch of
  *           `nsys` same-shape systems stores system s at offset s*(that size).
+ *           A_i is symmetric, and only its upper triangle (row <= column) is read.
  * Precision: dtype BSS_F64 / BSS_F32 for plain solves in that precision; mode
  *           BSS_MODE_MIXED (dtype must be BSS_F64) factors in FP32 on MFMA and
  *           refines in FP64 to a normwise backward error target.

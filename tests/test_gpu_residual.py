@@ -51,7 +51,7 @@ def berr_extended(A, B, x, d):
     return (np.abs(r).max(axis=(0, 1)) / den).astype(np.float64)
 
 
-@pytest.mark.parametrize("nrhs", [1])
+@pytest.mark.parametrize("nrhs", [1, 3, 16])
 @pytest.mark.parametrize("N", [1, 2, 3, 6, 32, 33, 71])
 @pytest.mark.parametrize("n", [16, 32, 48, 64, 96, 128])
 def test_residual(n, N, nrhs):
