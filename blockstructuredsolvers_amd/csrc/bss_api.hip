@@ -1325,13 +1325,19 @@ int bss_factorize_solve(bss_plan_t p, void* stream) {
   p->fsweep_pending = false;
   p->info_valid = false;
   p->fb_active = p->fb_factored = false;
-  if (!p->side_stream) {
+  // Up to n = 32 a level's sweep (4-6 us) takes less than the event record and the two waits
+  // that hand it to a second stream: everything in the caller's order was faster at every
+  // length (smoother requests, n = 16: 167 -> 143 us at N = 128, 241 -> 215 at N = 4096; n =
+  // 32: 213 -> 200 and 361 -> 349), and from n = 48 on slower (n = 64, N = 4096: 1044 ->
+  // 1113 us; n = 96, N = 300: 687 -> 724).
+  const bool side = p->n > 32;
+  if (side && !p->side_stream) {
     HIP_TRY(hipStreamCreateWithFlags(&p->side_stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreateWithFlags(&p->ev_l0_factored, hipEventDisableTiming));
     HIP_TRY(hipEventCreateWithFlags(&p->ev_l0_solved, hipEventDisableTiming));
   }
   const size_t L = p->gl.size();
-  while (p->ev_level.size() < L) {
+  while (side && p->ev_level.size() < L) {
     hipEvent_t ev;
     HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     p->ev_level.push_back(ev);
@@ -1359,9 +1365,11 @@ int bss_factorize_solve(bss_plan_t p, void* stream) {
   // beside the later, latency-bound levels.
   const size_t split = 2;
   if (int e = factor(0, split)) return e;
-  hipStream_t s2 = p->side_stream;
-  HIP_TRY(hipEventRecord(p->ev_l0_factored, s));
-  HIP_TRY(hipStreamWaitEvent(s2, p->ev_l0_factored, 0));
+  hipStream_t s2 = side ? p->side_stream : s;
+  if (side) {
+    HIP_TRY(hipEventRecord(p->ev_l0_factored, s));
+    HIP_TRY(hipStreamWaitEvent(s2, p->ev_l0_factored, 0));
+  }
   // side stream: the first solve's forward sweeps of the factored levels beside the
   // later levels' factorisation
   if (mixed && !fuse && bss::mixed_first_pass(p->mx, hooks, s2) != 0)
@@ -1380,9 +1388,11 @@ int bss_factorize_solve(bss_plan_t p, void* stream) {
   for (size_t l = split; l < L && rc == BSS_OK && e == hipSuccess; ++l) {
     rc = factor(l, l + 1);
     if (rc != BSS_OK) break;
-    e = hipEventRecord(p->ev_level[l], s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(s2, p->ev_level[l], 0);
-    if (e != hipSuccess) break;
+    if (side) {
+      e = hipEventRecord(p->ev_level[l], s);
+      if (e == hipSuccess) e = hipStreamWaitEvent(s2, p->ev_level[l], 0);
+      if (e != hipSuccess) break;
+    }
     GLevel& G = p->gl[l];
     const bss::SolveLevelArgs a{G.dchains, G.dtab[0], p->nrhs};
     ProfScope ps(p, BSS_K_FORWARD, (int)l, s2);
@@ -1399,8 +1409,8 @@ int bss_factorize_solve(bss_plan_t p, void* stream) {
   }
   // the join is recorded and awaited even after a failure, so that the caller's stream
   // never runs ahead of side-stream work
-  const hipError_t ej = hipEventRecord(p->ev_l0_solved, s2);
-  if (ej == hipSuccess) HIP_TRY(hipStreamWaitEvent(s, p->ev_l0_solved, 0));
+  const hipError_t ej = side ? hipEventRecord(p->ev_l0_solved, s2) : hipSuccess;
+  if (side && ej == hipSuccess) HIP_TRY(hipStreamWaitEvent(s, p->ev_l0_solved, 0));
   if (e != hipSuccess) return fail(BSS_E_HIP, "side-stream forward sweep: %s", hipGetErrorString(e));
   if (ej != hipSuccess) return fail(BSS_E_HIP, "side-stream join: %s", hipGetErrorString(ej));
   if (rc != BSS_OK) return rc;

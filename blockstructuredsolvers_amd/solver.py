@@ -605,9 +605,11 @@ def build_smoother(data: BlockTriDiagData_batched, model) -> None:
     if model.F.shape != (n, n):
         raise ValueError(f"model state size {model.F.shape} does not match n={n}")
     dev = data.device
-    # column-major device copies: the row-major storage of M^T is M column by column
-    F, H, Qi, Ri = [torch.from_numpy(np.ascontiguousarray(np.asarray(M, dtype=np.float64).T)).to(dev)
-                    for M in (model.F, model.H, model.Qinv, model.Rinv)]
+    # column-major, one after the other: one copy to the device (four took 45 us each)
+    parts = [np.asarray(M, dtype=np.float64).ravel(order="F")
+             for M in (model.F, model.H, model.Qinv, model.Rinv)]
+    buf = torch.from_numpy(np.concatenate(parts)).pin_memory().to(dev, non_blocking=True)
+    F, H, Qi, Ri = torch.split(buf, [p.size for p in parts])
     code = L.BSS_F64 if data.dtype == torch.float64 else L.BSS_F32
     with torch.cuda.device(dev):
         L.call("bss_build_smoother", data.n_user, n, model.H.shape[0], F.data_ptr(),
