@@ -86,8 +86,8 @@ template <typename Tin, typename Ts, typename To>
 hipError_t launch_assemble_diag(const SepRec* seps, const LevelSys* sys, int nb, int nsep,
                                 hipStream_t s) {
   if (nsep <= 0) return hipSuccess;
-  hipLaunchKernelGGL((assemble_diag_kernel<Tin, Ts, To>), dim3(nsep), dim3(256), 0, s, seps, sys,
-                     nb * nb);
+  hipLaunchKernelGGL((assemble_diag_kernel<Tin, Ts, To>), dim3(nsep, nb / 16), dim3(256), 0, s,
+                     seps, sys, nb);
   return hipGetLastError();
 }
 

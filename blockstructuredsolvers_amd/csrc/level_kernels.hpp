@@ -15,24 +15,38 @@
 
 namespace bss {
 
-// One workgroup per separator (all systems of the level in one launch).  Ts is the
-// element type of the chain contributions and of this level's vectors, To that of the
-// next level; they differ only at the hand-off from an FP32 level to FP64 separator
-// levels (mixed mode after a separator re-factorisation).
+// One workgroup per separator and 16-column strip (all systems of the level in one launch),
+// upper tiles only: a thread has one entry of each, and their loads are in flight together
+// (one workgroup walking the whole block one entry a thread at a time took 28 us at n = 128
+// with a handful of separators, and 223 for 2047, 1.3 GB; this takes 5 and 130).  Ts is the
+// element type of the chain contributions, To that of the next level; they differ only at
+// the hand-off from an FP32 level to FP64 separator levels (mixed mode after a separator
+// re-factorisation).
 template <typename Tin, typename Ts, typename To>
 __global__ void __launch_bounds__(256) assemble_diag_kernel(const SepRec* __restrict__ seps,
                                                              const LevelSys* __restrict__ sys,
-                                                             int nn) {
+                                                             int nb) {
   const SepRec sr = seps[blockIdx.x];
   const LevelSys& S = sys[sr.slot];
-  const auto a = gptr((const Tin*)S.A) + (long long)sr.pos * nn;
-  const auto r = gptr((const Ts*)S.SR) + (long long)sr.p * nn;
-  const auto l = gptr((const Ts*)S.SL) + (long long)sr.p * nn;
-  const auto an = gptr((To*)S.An) + (long long)sr.p * nn;
-  for (int e = threadIdx.x; e < nn; e += blockDim.x) {
-    const double v = (double)a[e] - (double)r[e] - (double)l[e];
-    an[e] = (To)v;
+  const long long nn = (long long)nb * nb;
+  const int b = blockIdx.y, e0 = (16 * b + (threadIdx.x >> 4)) * nb + (threadIdx.x & 15);
+  const auto a = gptr((const Tin*)S.A) + (long long)sr.pos * nn + e0;
+  const auto r = gptr((const Ts*)S.SR) + (long long)sr.p * nn + e0;
+  const auto l = gptr((const Ts*)S.SL) + (long long)sr.p * nn + e0;
+  const auto an = gptr((To*)S.An) + (long long)sr.p * nn + e0;
+  constexpr int MAXT = 8;  // n <= 128
+  double v[MAXT][3];
+#pragma unroll
+  for (int t = 0; t < MAXT; ++t) {
+    if (t <= b) {
+      v[t][0] = (double)a[16 * t];
+      v[t][1] = (double)r[16 * t];
+      v[t][2] = (double)l[16 * t];
+    }
   }
+#pragma unroll
+  for (int t = 0; t < MAXT; ++t)
+    if (t <= b) an[16 * t] = (To)(v[t][0] - v[t][1] - v[t][2]);
 }
 
 template <typename Ts, typename To>
