@@ -127,6 +127,7 @@ struct bss_plan {
   std::vector<int> chain_len = std::vector<int>(16, 0);  // per-level overrides
   int chain_len_default = 3;
   int base_max = 8;
+  bool lens_given = false;  // any of these three set: the others keep their defaults
   bool preserve = true;  // plain mode: factors to workspace, A/B untouched
   // bss_info: per-system LAPACK-order info of the last factorisation, computed once
   std::vector<int> info_exact;
@@ -270,6 +271,10 @@ struct Bump {
 std::vector<bss::LevelShape> schedule_of(const bss_plan* p, int N, int* n_use) {
   if (p->schedule == BSS_SCHED_REFERENCE) return bss::reference_schedule_levels(N, n_use);
   *n_use = N;
+  if (!p->lens_given) {
+    const bss::ChainLens a = bss::auto_chain_lens(N, p->n);
+    return bss::auto_schedule(N, {a.first}, a.rest, a.base);
+  }
   return bss::auto_schedule(N, p->chain_len, p->chain_len_default, std::max(1, p->base_max));
 }
 
@@ -925,6 +930,7 @@ int fallback_solve(bss_plan* p, hipStream_t s) {
     q->chain_len = p->chain_len;
     q->chain_len_default = p->chain_len_default;
     q->base_max = p->base_max;
+    q->lens_given = p->lens_given;
     q->preserve = true;
     if (int e = bss_plan_bind(q, p->A, p->B, x0)) {
       bss_plan_destroy(q);
@@ -984,6 +990,7 @@ int sequential_info(bss_plan* p, int s, hipStream_t st, int* out) {
   bss_plan* q = nullptr;
   if (int e = create(1, &NU, p->n, 1, dt, BSS_MODE_PLAIN, BSS_SCHED_AUTO, &q)) return e;
   q->base_max = NU;  // one level: a single chain over all blocks
+  q->lens_given = true;
   q->preserve = true;
   // the chain's factorisation reads A and B only; d is bound because a plan needs one
   int rc = bss_plan_bind(q, (char*)p->A + oa * is,
@@ -1153,6 +1160,7 @@ int bss_set_option(bss_plan_t p, int option, double value) {
     case BSS_OPT_CHAIN_LEN:
       if (value < 1 || value > 1 << 20) return fail(BSS_E_ARG, "chain length must be >= 1");
       p->chain_len_default = (int)value;
+      p->lens_given = true;
       return BSS_OK;
     case BSS_OPT_FACTOR_WAVES:
       if (value != 4 && value != 8) return fail(BSS_E_ARG, "factor waves must be 4 or 8");
@@ -1165,6 +1173,7 @@ int bss_set_option(bss_plan_t p, int option, double value) {
     case BSS_OPT_BASE_MAX:
       if (value < 1 || value > 1 << 20) return fail(BSS_E_ARG, "base_max must be >= 1");
       p->base_max = (int)value;
+      p->lens_given = true;
       return BSS_OK;
     case BSS_OPT_PRESERVE_INPUT:
       p->preserve = value != 0.0;
@@ -1190,6 +1199,7 @@ int bss_set_option(bss_plan_t p, int option, double value) {
       if (option >= BSS_OPT_CHAIN_LEN_LEVEL && option < BSS_OPT_CHAIN_LEN_LEVEL + 16) {
         if (value < 1 || value > 1 << 20) return fail(BSS_E_ARG, "chain length must be >= 1");
         p->chain_len[option - BSS_OPT_CHAIN_LEN_LEVEL] = (int)value;
+        p->lens_given = true;
         return BSS_OK;
       }
       return fail(BSS_E_ARG, "unknown option %d", option);

@@ -116,6 +116,28 @@ inline LevelShape split_level(int N, int m) {
   return L;
 }
 
+// Chain lengths (first level, the others) and largest base level where none is given.
+struct ChainLens {
+  int first, rest, base;
+};
+// Longer level-0 chains leave fewer separators (less factor, panel and sweep work at every
+// later level), as long as one system alone still has a chain per CU: N / 256 - 1 blocks,
+// up to a length from which the chain's own latency costs more than the levels it saves --
+// the earlier, the smaller the blocks, whose chains share a CU several at a time.  They do
+// not depend on how many systems a plan has, so a system's answer does not either.
+// Factorize and solve in FP64, one system, in us, with chains of 3 at every level against
+// these: n = 16, N = 2048: 141 -> 135; n = 32, 8192: 375 -> 333; n = 64, 2048: 509 -> 479,
+// 8192: 1125 -> 988; n = 128, 2048: 2310 -> 2100, 8192: 5563 -> 4886 (eight systems of 8192
+// blocks at n = 96: 18059 -> 16701).  From n = 64 on a level costs less than a block more in
+// each of its chains, so the later levels take chains of two and a base of four (n = 128, N =
+// 8192: 5082 with three and eight).  Below N = 1280 chains of three are as good or better
+// (n = 64, N = 512: 357, with seven 373), and need no more workspace.
+inline ChainLens auto_chain_lens(int N, int n) {
+  const int m = std::min(N / 256 - 1, n <= 32 ? 7 : n <= 64 ? 15 : 31);
+  if (m <= 3) return {3, 3, 8};
+  return n >= 64 ? ChainLens{m, 2, 4} : ChainLens{m, 3, 8};
+}
+
 // Full schedule: levels top first, the last one a single chain.
 // chain_len[k] > 0 fixes level k's chain length; other levels use `m_default`.
 inline std::vector<LevelShape> auto_schedule(int N, const std::vector<int>& chain_len,
