@@ -1,8 +1,7 @@
 """Schedule autotuner for libbss plans.
 
 A plan's speed depends on its level schedule (chain length per level, size of the
-single-chain base level) and, at n = 64, on the factor workgroup size (4 or 8
-waves).  The reference fixes its schedule by an integer search
+single-chain base level).  The reference fixes its schedule by an integer search
 (src/gpu_batched.jl:112-162); here candidates are timed on the device and the fastest
 is cached in ``tuned.json`` next to this file.
 
@@ -70,14 +69,10 @@ def lookup(N: int, n: int, dtype, mode: str, path: str = CACHE, nsys: int = 1) -
 
 def candidates(n: int, nsys: int = 1) -> List[dict]:
     """Top-level chain lengths up to 63 (long chains pay when many systems share the
-    plan), lower levels 2-4, base 2-8; at n = 64 both factor workgroup sizes (one
-    system) or 8 waves (batches, where 8 won every earlier tune)."""
-    waves = ([4, 8] if nsys == 1 else [8]) if n == 64 else [None]
+    plan), lower levels 2-4, base 2-8."""
     out = []
-    for w, top, low, base in itertools.product(waves, [2, 3, 4, 6, 7, 15, 31, 63], [2, 3, 4],
-                                               [2, 4, 8]):
-        out.append({"factor_waves": w, "chain_len_levels": [top] + [low] * 15,
-                    "base_max": base})
+    for top, low, base in itertools.product([2, 3, 4, 6, 7, 15, 31, 63], [2, 3, 4], [2, 4, 8]):
+        out.append({"chain_len_levels": [top] + [low] * 15, "base_max": base})
     return out
 
 
