@@ -48,19 +48,45 @@ hipError_t launch_factor(int nb, const FactorLevelArgs& a, int nchains, hipStrea
   }
 }
 
+// One right-hand side on vector FMAs; several on MFMA, in FP64 one kernel up to 4, 8 and 16
+// (RhsTile; a column's bits are the same in each)
+template <typename T, int NB>
+static hipError_t forward_nb(const SolveLevelArgs& a, int nchains, hipStream_t s) {
+  const dim3 grid(nchains), block(4 * NB);
+  if (a.nrhs == 1)
+    hipLaunchKernelGGL((chain_forward1_kernel<T, NB>), grid, block, 0, s, a);
+  else if (sizeof(T) == 8 && a.nrhs <= 4)
+    hipLaunchKernelGGL((chain_forward_kernel<T, NB, sizeof(T) == 8 ? 1 : 4>), grid, block, 0, s, a);
+  else if (sizeof(T) == 8 && a.nrhs <= 8)
+    hipLaunchKernelGGL((chain_forward_kernel<T, NB, sizeof(T) == 8 ? 2 : 4>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((chain_forward_kernel<T, NB, 4>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+template <typename T, int NB>
+static hipError_t backward_nb(const SolveLevelArgs& a, int nchains, hipStream_t s) {
+  const dim3 grid(nchains), block(4 * NB);
+  if (a.nrhs == 1)
+    hipLaunchKernelGGL((chain_backward1_kernel<T, NB>), grid, block, 0, s, a);
+  else if (sizeof(T) == 8 && a.nrhs <= 4)
+    hipLaunchKernelGGL((chain_backward_kernel<T, NB, sizeof(T) == 8 ? 1 : 4>), grid, block, 0, s, a);
+  else if (sizeof(T) == 8 && a.nrhs <= 8)
+    hipLaunchKernelGGL((chain_backward_kernel<T, NB, sizeof(T) == 8 ? 2 : 4>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((chain_backward_kernel<T, NB, 4>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_forward(int nb, const SolveLevelArgs& a, int nchains, hipStream_t s) {
   if (nchains <= 0) return hipSuccess;
   switch (nb) {
-#define BSS_FWD(NB)                                                                          \
-  case NB:                                                                                   \
-    if (a.nrhs == 1)                                                                         \
-      hipLaunchKernelGGL((chain_forward1_kernel<T, NB>), dim3(nchains), dim3(4 * NB), 0, s, a); \
-    else                                                                                     \
-      hipLaunchKernelGGL((chain_forward_kernel<T, NB>), dim3(nchains), dim3(4 * NB), 0, s, a); \
-    return hipGetLastError();
-    BSS_FWD(16) BSS_FWD(32) BSS_FWD(48) BSS_FWD(64) BSS_FWD(96) BSS_FWD(128)
-#undef BSS_FWD
+    case 16: return forward_nb<T, 16>(a, nchains, s);
+    case 32: return forward_nb<T, 32>(a, nchains, s);
+    case 48: return forward_nb<T, 48>(a, nchains, s);
+    case 64: return forward_nb<T, 64>(a, nchains, s);
+    case 96: return forward_nb<T, 96>(a, nchains, s);
+    case 128: return forward_nb<T, 128>(a, nchains, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -69,15 +95,12 @@ template <typename T>
 hipError_t launch_backward(int nb, const SolveLevelArgs& a, int nchains, hipStream_t s) {
   if (nchains <= 0) return hipSuccess;
   switch (nb) {
-#define BSS_BWD(NB)                                                                           \
-  case NB:                                                                                    \
-    if (a.nrhs == 1)                                                                          \
-      hipLaunchKernelGGL((chain_backward1_kernel<T, NB>), dim3(nchains), dim3(4 * NB), 0, s, a); \
-    else                                                                                      \
-      hipLaunchKernelGGL((chain_backward_kernel<T, NB>), dim3(nchains), dim3(4 * NB), 0, s, a); \
-    return hipGetLastError();
-    BSS_BWD(16) BSS_BWD(32) BSS_BWD(48) BSS_BWD(64) BSS_BWD(96) BSS_BWD(128)
-#undef BSS_BWD
+    case 16: return backward_nb<T, 16>(a, nchains, s);
+    case 32: return backward_nb<T, 32>(a, nchains, s);
+    case 48: return backward_nb<T, 48>(a, nchains, s);
+    case 64: return backward_nb<T, 64>(a, nchains, s);
+    case 96: return backward_nb<T, 96>(a, nchains, s);
+    case 128: return backward_nb<T, 128>(a, nchains, s);
     default: return hipErrorInvalidValue;
   }
 }
