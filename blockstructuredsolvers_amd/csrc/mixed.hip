@@ -70,23 +70,21 @@ __global__ void __launch_bounds__(kRedThreads)
 // 16 blocks each; 24 or 64 blocks were 30% slower)
 int blocks_per_item(int N) { return std::max(32, (N + 255) / 256); }
 
-// The first pass of a solve (x = 0, so r = d): d into the FP32 vector, zeros into the
-// FP64 iterate, and the item's per-column max |d_j| (as both the residual and the
+// The first pass of a solve (x = 0, so r = d): d into the FP32 vector (the iterate is not
+// written: the first residual pass takes it as zero), and the item's per-column max |d_j| (as both the residual and the
 // right-hand-side maxima; the iterate maximum is 0).  Elementwise, with no block
 // window: one workgroup per residual work item, kInitThreads threads.
 constexpr int kInitThreads = 256;
 
 __global__ void __launch_bounds__(kInitThreads)
     init_pass_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
-                     double* __restrict__ part, int n, int nrhs, int xn_k, int ro_k,
-                     const int* __restrict__ skip) {
+                     double* __restrict__ part, int n, int nrhs, int ro_k, const int* __restrict__ skip) {
   __shared__ double red[kInitThreads / 64];
   if (skip && *skip == 0) return;  // the whole workgroup leaves (uniform)
   const ResItem it = items[blockIdx.x];
   const ResSys& S = systems[it.sys];
   const long long ND = (long long)n * nrhs;
   const auto ds = gptr(S.d);
-  const auto xn = gptr(S.x[xn_k]);
   const auto ro = gptr(S.v[ro_k]);
   const int tid = threadIdx.x, w = wave_id(), l = lane_id();
   const int per = kInitThreads / n;  // blocks per sweep of the workgroup (n <= 128)
@@ -97,7 +95,6 @@ __global__ void __launch_bounds__(kInitThreads)
       const long long e = j * ND + (long long)c * n + tid % n;
       const double v = ds[e];
       ro[e] = (float)v;
-      xn[e] = 0.0;
       m = nmax(m, fabs(v));
     }
 #pragma unroll
@@ -116,24 +113,34 @@ __global__ void __launch_bounds__(kInitThreads)
   if (tid == 0) out[kMnormSlot] = 0.0;
 }
 
+// xo_k < 0: the iterate is zero
+template <int NB, bool X0>
+void launch_residual_nb(const MixedState& m, int xo_k, int dx_k, int xn_k, int ro_k,
+                        int want_mnorm, hipStream_t s) {
+  const dim3 grid(m.nitems), block(64 * kColWaves);
+  if (m.nrhs == 1 && !want_mnorm)
+    hipLaunchKernelGGL((residual_column_kernel<NB, false, X0>), grid, block, 0, s, m.items,
+                       m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
+  else if (m.nrhs == 1)
+    hipLaunchKernelGGL((residual_column_kernel<NB, true, X0>), grid, block, 0, s, m.items,
+                       m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
+  else if (!want_mnorm)
+    hipLaunchKernelGGL((residual_tiles_kernel<NB, false, X0>), grid, block, 0, s, m.items,
+                       m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
+  else
+    hipLaunchKernelGGL((residual_tiles_kernel<NB, true, X0>), grid, block, 0, s, m.items,
+                       m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
+}
 template <int NB>
 hipError_t launch_residual(const MixedState& m, bool init, int xo_k, int dx_k, int xn_k,
                            int ro_k, int want_mnorm, hipStream_t s) {
   if (init)
     hipLaunchKernelGGL(init_pass_kernel, dim3(m.nitems), dim3(kInitThreads), 0, s, m.items,
-                       m.sys_dev, m.part, NB, m.nrhs, xn_k, ro_k, m.init_skip);
-  else if (m.nrhs == 1 && !want_mnorm)
-    hipLaunchKernelGGL((residual_column_kernel<NB, false>), dim3(m.nitems), dim3(64 * kColWaves),
-                       0, s, m.items, m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
-  else if (m.nrhs == 1)
-    hipLaunchKernelGGL((residual_column_kernel<NB, true>), dim3(m.nitems), dim3(64 * kColWaves),
-                       0, s, m.items, m.sys_dev, m.part, xo_k, dx_k, xn_k, ro_k);
-  else if (!want_mnorm)
-    hipLaunchKernelGGL((residual_tiles_kernel<NB, false>), dim3(m.nitems), dim3(64 * kColWaves),
-                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
+                       m.sys_dev, m.part, NB, m.nrhs, ro_k, m.init_skip);
+  else if (xo_k < 0)
+    launch_residual_nb<NB, true>(m, xo_k, dx_k, xn_k, ro_k, want_mnorm, s);
   else
-    hipLaunchKernelGGL((residual_tiles_kernel<NB, true>), dim3(m.nitems), dim3(64 * kColWaves),
-                       0, s, m.items, m.sys_dev, m.part, m.nrhs, xo_k, dx_k, xn_k, ro_k);
+    launch_residual_nb<NB, false>(m, xo_k, dx_k, xn_k, ro_k, want_mnorm, s);
   return hipGetLastError();
 }
 
@@ -409,7 +416,7 @@ int mixed_solve(MixedState& m, const MixedSolveHooks& h, double* d, double tol, 
       }
     }
     const int want_mnorm = m.mnorm_stale ? 1 : 0;
-    e = residual_prof(m, h, false, xa, cur, 1 - xa, 1 - cur, want_mnorm, s);
+    e = residual_prof(m, h, false, it == 0 ? -1 : xa, cur, 1 - xa, 1 - cur, want_mnorm, s);
     m.mnorm_stale = false;
     if (e != hipSuccess) {
       g_mixed_err = hipGetErrorString(e);

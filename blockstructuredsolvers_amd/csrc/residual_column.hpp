@@ -93,7 +93,8 @@ constexpr int kColWaves = 4;  // waves of a work-group: block rows of an item in
 // 2.69; 8 systems of 2048 blocks, n = 96: 0.50 -> 0.37 ms, with ||M|| 0.53 -> 0.38.
 // Eight waves a work-group at 128 registers spill; four at 168 give the same bytes in
 // flight.
-template <int NB, bool MN>
+// X0: x_old is zero (the first pass of a solve), and neither read nor there.
+template <int NB, bool MN, bool X0>
 __global__ void __launch_bounds__(64 * kColWaves)
     __attribute__((amdgpu_waves_per_eu(NB == 96 && MN ? 2 : 3)))  // (LDS: two work-groups a CU)
     residual_column_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(64 * kColWaves)
   const auto As = gptr((const double*)S.A);
   const auto Bs = gptr((const double*)S.B);
   const auto ds = gptr((const double*)S.d);
-  const auto xo = gptr((const double*)S.x[xo_k]);
+  const auto xo = gptr((const double*)(X0 ? nullptr : S.x[xo_k]));
   const auto dxs = gptr((const float*)S.v[dx_k]);
   const auto xn = gptr(S.x[xn_k]);
   const auto ro = gptr(S.v[ro_k]);
@@ -144,7 +145,9 @@ __global__ void __launch_bounds__(64 * kColWaves)
   };
   auto load_x = [&](int j) -> xv_t {  // clamped: every load is unconditional
     const long long e = (long long)(j < 0 ? 0 : j >= N ? N - 1 : j) * NB + 2 * q;
-    return xv_t{*(const BSS_GLOBAL d2_t*)(xo + e), *(const BSS_GLOBAL f2_t*)(dxs + e)};
+    const f2_t d = *(const BSS_GLOBAL f2_t*)(dxs + e);
+    if constexpr (X0) return xv_t{d2_t{0.0, 0.0}, d};
+    else return xv_t{*(const BSS_GLOBAL d2_t*)(xo + e), d};
   };
   auto sum_x = [&](const xv_t& v, int j) -> l2_t {
     const bool in = j >= 0 && j < N;

@@ -19,7 +19,13 @@ template <int NB, bool MN>
 struct RowTiles {
   static constexpr int TT = NB / 16;
   static constexpr int NA = TT * (TT + 1) / 2, T = NA + TT * TT;
-  static constexpr int RING = NB == 16 ? 2 : NB == 32 ? 4 : NB == 48 ? 5 : NB == 64 ? (MN ? 4 : 5) : NB == 96 ? 10 : MN ? 5 : 8;
+  static constexpr int RING = NB == 16   ? 2
+                              : NB == 32 ? 4
+                              : NB == 48 ? 5
+                              : NB == 64 ? (MN ? 4 : 5)
+                              : NB == 96 ? 10
+                              : MN       ? 5
+                                         : 8;
   static constexpr int STEPS = (T + RING - 1) / RING * RING;
   static constexpr bool is_a(int s) { return s < NA; }
   static constexpr int col(int s) {
@@ -60,7 +66,8 @@ __device__ __attribute__((always_inline)) inline void for_each_step(
 // Measured against a work-group per block row (two barriers a row, B read a second time as
 // transposed operand, A read whole), 8 systems of 4096 blocks, n = 64, 16 right-hand sides:
 // 712 -> 604 us, 2.8 GB at 4.6 TB/s (a copy reaches 4.9, reads alone 6.1).
-template <int NB, bool MN>
+// X0: x_old is zero (the first pass of a solve), and neither read nor there.
+template <int NB, bool MN, bool X0>
 __global__ void __launch_bounds__(64 * kColWaves)
     __attribute__((amdgpu_waves_per_eu(RowTiles<NB, MN>::waves_per_eu())))
     residual_tiles_kernel(const ResItem* __restrict__ items, const ResSys* __restrict__ systems,
@@ -89,7 +96,7 @@ __global__ void __launch_bounds__(64 * kColWaves)
   const auto As = gptr((const double*)S.A);
   const auto Bs = gptr((const double*)S.B);
   const auto ds = gptr((const double*)S.d);
-  const auto xo = gptr((const double*)S.x[xo_k]);
+  const auto xo = gptr((const double*)(X0 ? nullptr : S.x[xo_k]));
   const auto dxs = gptr((const float*)S.v[dx_k]);
   const auto xn = gptr(S.x[xn_k]);
   const auto ro = gptr(S.v[ro_k]);
@@ -117,8 +124,10 @@ __global__ void __launch_bounds__(64 * kColWaves)
     for (int t = 0; t < TT; ++t) {
       v.d[t] = *(const BSS_GLOBAL f4u_t*)at(dxs + e + 16 * t, 4 * xl);
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        v.o[t][h] = *(const BSS_GLOBAL d2_t*)at(xo + e + 16 * t + 2 * h, 8 * xl);
+      for (int h = 0; h < 2; ++h) {
+        if constexpr (X0) v.o[t][h] = d2_t{0.0, 0.0};
+        else v.o[t][h] = *(const BSS_GLOBAL d2_t*)at(xo + e + 16 * t + 2 * h, 8 * xl);
+      }
     }
   };
   auto neg_x = [&](double(&nx)[TT][4], const xraw_t& v, int j) {
