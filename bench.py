@@ -272,11 +272,12 @@ def roofline_for(res, args, nsys):
         # leaves at once (one per step), so the rate is over the launches that swept
         count = max(count - res.get("profiled_steps", 0), 1)
     avg_ms = total / count
+    tri = n * (n + 1) // 2
     if name == "factor":
         s_in = 8 if level == 0 else sf
-        # algorithmic: read A, B; write U, C (4 N n^2 s, with input/factor sizes); with the
-        # fused level-0 forward sweep also read r and write y (2 n nrhs sf)
-        bytes_per = 2 * n * n * s_in + 2 * n * n * sf + (2 * n * nrhs * sf if fused else 0)
+        # algorithmic: read A's triangle and B; write U's triangle and C; with the fused
+        # level-0 forward sweep also read r and write y (2 n nrhs sf)
+        bytes_per = (tri + n * n) * (s_in + sf) + (2 * n * nrhs * sf if fused else 0)
         flops_per = 7.0 / 3.0 * n ** 3
         alg_bytes = blocks * bytes_per
         alg_flops = blocks * flops_per
@@ -290,11 +291,11 @@ def roofline_for(res, args, nsys):
                         per_launch_ms=avg_ms, launches=count)
     elif name in ("forward", "backward"):
         # read Uinv (upper triangle), C, W and the vectors; write the vectors
-        tri = n * (n + 1) // 2
         bytes_per = (tri + 2 * n * n) * sf + 2 * n * nrhs * sf
         alg_bytes = blocks * bytes_per
     elif name == "residual":
-        bytes_per = 2 * n * n * 8 + n * nrhs * (8 * 3 + 4 * 2)
+        # read A's triangle, B and the vectors; write the vectors
+        bytes_per = (tri + n * n) * 8 + n * nrhs * (8 * 3 + 4 * 2)
         alg_bytes = NL * nsys * bytes_per
     else:
         alg_bytes = 0

@@ -126,9 +126,8 @@ def tune(N: int, n: int, nrhs: int = 1, dtype=torch.float64, mode: str = "plain"
     results.sort(key=lambda t: t[0])
     best_ms, best = results[0]
     entry = {"config": best, "ms": best_ms,
-             "default_ms": next((m for m, c in results if c.get("factor_waves", 4) == 4 and
-                                 c["chain_len_levels"][0] == 3 and c["chain_len_levels"][1] == 3
-                                 and c["base_max"] == 8), None)}
+             "default_ms": next((m for m, c in results if c["chain_len_levels"][0] == 3 and
+                                 c["chain_len_levels"][1] == 3 and c["base_max"] == 8), None)}
     if save:
         cache = load_cache(path)
         cache[key(N, n, dtype, mode, nsys)] = entry

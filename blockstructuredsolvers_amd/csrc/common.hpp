@@ -163,10 +163,10 @@ __device__ inline void atomic_max_nonneg(unsigned long long* addr, double v) {
 }
 
 // Whether a level's forward sweep runs in the factor kernel (FactorLevelArgs::fwd): FP32
-// factors on the LDS kernel (n <= 64 and n = 96), one right-hand side.  With FP64
-// factors the fused kernel is at its register limit and spills; measured at N = 8192,
-// n = 64 (16 systems) its level-0 factor took 11.1 ms instead of 9.5, more than the
-// separate sweep it saves (FP32: 4.82 instead of 4.74 ms, saving a 1.0 ms sweep).
+// factors up to n = 96, one right-hand side.  Mixed factorize and solve, sweep in a launch of
+// its own against fused: 32 systems of 8192 blocks, n = 64, 20.88 -> 19.17 ms; 8 of 4096, n =
+// 48, 1.88 -> 1.76; 4 of 8192, n = 96, 7.99 -> 7.62.  With FP64 factors the strips leave it no
+// registers (230 of 256 at n = 64, all at n = 96).
 inline bool factor_fuses_forward(int nb, bool fp32_factors, int nrhs) {
   return nrhs == 1 && fp32_factors && (nb == 16 || nb == 32 || nb == 48 || nb == 64 || nb == 96);
 }
