@@ -60,10 +60,6 @@ __device__ inline int opaque_v(int x) {
   asm volatile("" : "+v"(x));
   return x;
 }
-__device__ inline int opaque_s(int x) {
-  asm volatile("" : "+s"(x));
-  return x;
-}
 
 // Cross-lane helpers for the diagonal-tile routine.
 template <typename T>

@@ -77,17 +77,6 @@ __device__ inline double row4_sum(double t) {
 // unpredicated and the wait counters can be tracked exactly
 __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
-template <typename T>
-__device__ inline T rsqrt_t(T x);
-template <>
-__device__ inline double rsqrt_t<double>(double x) {
-  return 1.0 / sqrt(x);
-}
-template <>
-__device__ inline float rsqrt_t<float>(float x) {
-  return 1.0f / sqrtf(x);
-}
-
 // Pointers read from device tables are generic, and loads through them compile to FLAT
 // memory instructions, which count against the LDS wait counter as well: every wait for
 // an LDS read then also waits for all HBM loads in flight, defeating prefetches.
@@ -125,17 +114,6 @@ __device__ inline void tile_mma(typename Mfma<T>::acc_t& acc, PX __restrict__ xb
   }
 }
 
-// acc += op(X) op(Y) over K in 16-deep steps unrolled by two (not fully), which keeps
-// the operand registers of a full-depth product bounded
-template <typename T, bool TA, bool TB, bool NEG, int K, typename PX, typename PY>
-__device__ inline void tile_mma_k(typename Mfma<T>::acc_t& acc, PX __restrict__ xb, int ldx,
-                                  PY __restrict__ yb, int ldy) {
-#pragma unroll 2
-  for (int k0 = 0; k0 < K; k0 += 16)
-    tile_mma<T, TA, TB, NEG, 16>(acc, TA ? xb + k0 : xb + (long long)k0 * ldx, ldx,
-                                 TB ? yb + (long long)k0 * ldy : yb + k0, ldy);
-}
-
 // Load / store a D-layout tile from/to a column-major buffer (element (0,0) at p).
 template <typename T>
 __device__ inline typename Mfma<T>::acc_t tile_load(const T* p, int ld) {
@@ -153,13 +131,6 @@ __device__ inline void tile_store(T* p, int ld, const typename Mfma<T>::acc_t& a
   const int lr = l & 15, lk = l >> 4;
 #pragma unroll
   for (int v = 0; v < 4; ++v) p[lr * ld + Mfma<T>::row(lk, v)] = a[v];
-}
-
-// Order-independent max of non-negative doubles through their IEEE bit patterns
-// (non-negative doubles order like their uint64 encodings), so device-wide norm
-// reductions are deterministic.
-__device__ inline void atomic_max_nonneg(unsigned long long* addr, double v) {
-  atomicMax(addr, (unsigned long long)__double_as_longlong(v));
 }
 
 // Whether a level's forward sweep runs in the factor kernel (FactorLevelArgs::fwd): FP32
