@@ -164,11 +164,13 @@ __device__ inline double even_rows(double x) {
   return __hiloint2double((int)even_rows((unsigned)__double2hiint(x)),
                           (int)even_rows((unsigned)__double2loint(x)));
 }
-// x with lane L replaced by the wave-uniform v
+// x with lane L replaced by the wave-uniform v.  By the intrinsic (clang has no builtin for
+// it): two wait states have to lie between the lane read that writes v's SGPR and this read of
+// it, and the compiler keeps them only where it sees the instruction.
+__device__ int llvm_writelane(int v, int lane, int x) __asm("llvm.amdgcn.writelane.i32");
 template <int L>
 __device__ __attribute__((always_inline)) inline int write_lane(int x, int v) {
-  asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(__builtin_amdgcn_readfirstlane(v)), "n"(L));
-  return x;
+  return llvm_writelane(__builtin_amdgcn_readfirstlane(v), L, x);
 }
 template <int L>
 __device__ __attribute__((always_inline)) inline float write_lane(float x, float v) {
