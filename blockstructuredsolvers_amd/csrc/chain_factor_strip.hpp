@@ -185,12 +185,16 @@ __device__ __attribute__((always_inline)) inline double write_lane(double x, dou
 // Elimination steps of the 16x16 tile.  Every lane holds a column v[0..15]: in the even
 // 16-lane rows column c = lane % 16 of A, in the odd ones column c of the identity, which
 // becomes that of E.  Step J subtracts A[J][r] / A[J][J] times row J from the rows r > J
-// of both at once: m (row J of A in every 16-lane row) supplies the multipliers by DPP,
-// f = -v[J] / A[J][J] is the lane's own factor.  One FMA per row serves A and E (the same
-// steps on separate A and E registers take twice the FMAs, which a wave shares its SIMD's
-// issue slots for with the other waves' MFMAs).  Only the upper part of A is read.  The
-// scaling by 1 / sqrt of the pivots (gathered in pv) is left to the end.  The next step's
-// pivot chain is interleaved with this step's rows by hand: sched_barrier keeps the order.
+// of both at once: m (row J of A in every 16-lane row) supplies the multipliers by DPP, f
+// (row J, negated) is the lane's own factor.  Each of them takes 1 / sqrt of the pivot: 1 /
+// A[J][J] on one of them would be denormal for a pivot in the top binades (FP32's rcp returns
+// zero above 2^126), and takes 1% off a small FP64 system (n = 32, 100 blocks: 104.5 us, this
+// 105.7; powers of two formed on the scalar unit 110.5, tiles with such a diagonal scaled
+// under a branch 107.6).  One FMA per row serves A and E (the same steps on separate A and E
+// registers take twice the FMAs, which a wave shares its SIMD's issue slots for with the other
+// waves' MFMAs).  Only the upper part of A is read.  The scaling by 1 / sqrt of the pivots
+// (gathered in pv) is left to the end.  The next step's pivot chain is interleaved with this
+// step's rows by hand: sched_barrier keeps the order.
 template <int J>
 __device__ __attribute__((always_inline)) inline void elim_step(double (&v)[16], double m,
                                                                 double f, double& pv) {
@@ -202,15 +206,20 @@ __device__ __attribute__((always_inline)) inline void elim_step(double (&v)[16],
     fmac_rows<J + 2, J + 3>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
     const double p = read_lane(v[J + 1], J + 1);
-    const double mn = even_rows(v[J + 1]);
+    double mn = even_rows(v[J + 1]);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 3, J + 4>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const double y = __builtin_amdgcn_rcp(p);  // about 2^-24; third-order step below
+    const double y = __builtin_amdgcn_rsq(p);  // about 2^-24; third-order step below
     __builtin_amdgcn_sched_barrier(0);
-    fmac_rows<J + 4, J + 7>(v, m, f);
+    fmac_rows<J + 4, J + 6>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const double e = fma(-p, y, 1.0), g = v[J + 1] * y;
+    const double py = p * y;
+    __builtin_amdgcn_sched_barrier(0);
+    fmac_rows<J + 6, J + 7>(v, m, f);
+    __builtin_amdgcn_sched_barrier(0);
+    const double e = fma(-py, y, 1.0), g = v[J + 1] * y;
+    mn *= y;
     pv = write_lane<J + 1>(pv, p);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 7, J + 8>(v, m, f);
@@ -236,26 +245,33 @@ __device__ __attribute__((always_inline)) inline void elim_step(float (&v)[16], 
     fmac_rows<J + 2, J + 3>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
     const float p = read_lane(v[J + 1], J + 1);
-    const float mn = even_rows(v[J + 1]);
+    float mn = even_rows(v[J + 1]);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 3, J + 4>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const float y = __builtin_amdgcn_rcpf(p);  // 1 ulp, as the sweep's other roundings
+    const float y = __builtin_amdgcn_rsqf(p);  // 1 ulp, as the sweep's other roundings
     pv = write_lane<J + 1>(pv, p);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 4, J + 7>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
     const float fn = -(v[J + 1] * y);
+    mn *= y;
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 7, 16>(v, m, f);
     elim_step<J + 1>(v, mn, fn, pv);
   }
 }
-__device__ inline double neg_quot(double x, double p) {
-  const double y = __builtin_amdgcn_rcp(p), e = fma(-p, y, 1.0), g = x * y;
-  return fma(-g, fma(e, e, e), -g);
+// the first step's m and f from row 0
+__device__ inline void first_row(double x, double p, double& m, double& f) {
+  const double y = __builtin_amdgcn_rsq(p), e = fma(-(p * y), y, 1.0), g = x * y;
+  m = even_rows(x) * y;
+  f = fma(-g, fma(e, e, e), -g);
 }
-__device__ inline float neg_quot(float x, float p) { return -(x * __builtin_amdgcn_rcpf(p)); }
+__device__ inline void first_row(float x, float p, float& m, float& f) {
+  const float y = __builtin_amdgcn_rsqf(p);
+  m = even_rows(x) * y;
+  f = -(x * y);
+}
 template <int R, typename T>
 __device__ __attribute__((always_inline)) inline void scale_rows(T (&v)[16], T s) {
   if constexpr (R < 16) {
@@ -283,7 +299,9 @@ __device__ __attribute__((always_inline)) inline bool diag_img(const T* at, T* u
   }
   const T p = read_lane(v[0], 0);
   T pv = write_lane<0>(T(1), p);
-  elim_step<0>(v, even_rows(v[0]), neg_quot(v[0], p), pv);
+  T m, f;
+  first_row(v[0], p, m, f);
+  elim_step<0>(v, m, f, pv);
   __builtin_amdgcn_sched_barrier(0);
   scale_rows<0>(v, even_rows(rsqrt_nr(pv)));
   if ((lane_id() >> 4) == 1) {  // E[r][c] = Uinv[c][r] in v[r]
