@@ -507,7 +507,7 @@ def main():
     ap.add_argument("--base-max", type=int, default=None)
     ap.add_argument("--chain-lens", type=lambda v: [int(x) for x in v.split(",")], default=None,
                     help="per-level chain lengths, top level first")
-    ap.add_argument("--factor-waves", type=int, default=None)
+    ap.add_argument("--factor-waves", type=int, default=None, help="accepted, without effect")
     ap.add_argument("--graph", type=int, default=0, help="1: replay hipGraph-captured levels")
     ap.add_argument("--pivot-tol", type=float, default=None,
                     help="mixed: FP32 separator pivot threshold (2.0 forces the FP64 "

@@ -1164,7 +1164,6 @@ int bss_set_option(bss_plan_t p, int option, double value) {
       return BSS_OK;
     case BSS_OPT_FACTOR_WAVES:
       if (value != 4 && value != 8) return fail(BSS_E_ARG, "factor waves must be 4 or 8");
-      p->drop_graphs();
       return BSS_OK;
     case BSS_OPT_GRAPH:
       p->use_graph = value != 0.0;

@@ -308,8 +308,9 @@ def initialize_batched(N: int, n: int, T=torch.float64, M="cuda", *, nrhs: int =
     ``info()`` then gives a failing block that need not be the LAPACK-order first one);
     ``tol``/``max_iters`` control mixed-mode refinement and ``fallback`` (default on)
     its plain FP64 fallback when refinement stops short; ``chain_len``,
-    ``chain_len_levels``, ``base_max`` and ``factor_waves`` fix the auto schedule,
-    otherwise (``tuned=True``) it comes from the autotuner cache when one exists;
+    ``chain_len_levels`` and ``base_max`` fix the auto schedule, otherwise
+    (``tuned=True``) it comes from the autotuner cache when one exists;
+    ``factor_waves`` (4 or 8) is accepted without effect;
     ``graph=True`` replays each launch sequence from a captured hipGraph;
     ``pivot_tol`` (mixed) is the FP32 separator pivot threshold U_jj^2 / A_jj below
     which the separator levels are re-factored in FP64; ``torch_workspace`` takes the
@@ -320,7 +321,7 @@ def initialize_batched(N: int, n: int, T=torch.float64, M="cuda", *, nrhs: int =
     if device.type != "cuda":
         raise ValueError(f"M must name a GPU device, got {M!r}")
     if (tuned and schedule == "auto" and chain_len is None and base_max is None
-            and chain_len_levels is None and factor_waves is None):
+            and chain_len_levels is None):
         # schedule from the autotuner cache (keyed by N, n, type, mode and the largest
         # tuned batch-size bucket <= nsys)
         from .autotune import lookup
@@ -328,7 +329,6 @@ def initialize_batched(N: int, n: int, T=torch.float64, M="cuda", *, nrhs: int =
         if cfg:
             chain_len_levels = cfg.get("chain_len_levels")
             base_max = cfg.get("base_max")
-            factor_waves = cfg.get("factor_waves")
     return BlockTriDiagData_batched(N, n, T, device, nrhs, nsys, mode, schedule, chain_len,
                                     base_max, preserve_input, tol, max_iters,
                                     chain_len_levels, factor_waves, graph, pivot_tol,
@@ -400,13 +400,12 @@ def initialize_batched_group(Ns: List[int], n: int, T=torch.float64, M="cuda", *
     if device.type != "cuda":
         raise ValueError(f"M must name a GPU device, got {M!r}")
     if (tuned and schedule == "auto" and chain_len is None and base_max is None
-            and chain_len_levels is None and factor_waves is None):
+            and chain_len_levels is None):
         from .autotune import lookup
         cfgs = [lookup(N, n, T, mode, nsys=len(Ns)) for N in Ns]
         if cfgs[0] and all(c == cfgs[0] for c in cfgs):
             chain_len_levels = cfgs[0].get("chain_len_levels")
             base_max = cfgs[0].get("base_max")
-            factor_waves = cfgs[0].get("factor_waves")
     return BlockTriDiagData_group(list(Ns), n, T, device, nrhs, mode, schedule, chain_len,
                                   base_max, preserve_input, tol, max_iters, chain_len_levels,
                                   factor_waves, graph, pivot_tol, torch_workspace, fallback)
