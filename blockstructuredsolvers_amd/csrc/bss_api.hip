@@ -271,10 +271,7 @@ struct Bump {
 std::vector<bss::LevelShape> schedule_of(const bss_plan* p, int N, int* n_use) {
   if (p->schedule == BSS_SCHED_REFERENCE) return bss::reference_schedule_levels(N, n_use);
   *n_use = N;
-  if (!p->lens_given) {
-    const bss::ChainLens a = bss::auto_chain_lens(N, p->n);
-    return bss::auto_schedule(N, {a.first}, a.rest, a.base);
-  }
+  if (!p->lens_given) return bss::default_schedule(N, p->n);
   return bss::auto_schedule(N, p->chain_len, p->chain_len_default, std::max(1, p->base_max));
 }
 

@@ -92,13 +92,15 @@ inline LevelShape base_level(int N) {
   return L;
 }
 
+// The number of chains of about m blocks that a level of N blocks is split into.
+inline int chain_count(int N, int m) { return (N + 1 + (m + 1) / 2) / (m + 1); }
+
 // This library's schedule: Q chains whose lengths differ by at most one, the first and
 // last chains touching the ends of the level (so neither end is a separator and the
-// first chain carries no panel).  Q = round((N+1)/(m+1)); every chain has >= 1 block.
-inline LevelShape split_level(int N, int m) {
+// first chain carries no panel).  Every chain has >= 1 block.
+inline LevelShape split_level(int N, int Q) {
   LevelShape L;
   L.N = N;
-  int Q = (int)((N + 1 + (m + 1) / 2) / (m + 1));
   Q = std::max(2, std::min(Q, (N + 1) / 2));
   const int P = Q - 1;
   const int interior = N - P;
@@ -116,38 +118,18 @@ inline LevelShape split_level(int N, int m) {
   return L;
 }
 
-// Chain lengths (first level, the others) and largest base level where none is given.
-struct ChainLens {
-  int first, rest, base;
-};
-// Longer level-0 chains leave fewer separators (less factor, panel and sweep work at every
-// later level), as long as one system alone still has a chain per CU: N / 256 - 1 blocks,
-// up to a length from which the chain's own latency costs more than the levels it saves --
-// the earlier, the smaller the blocks, whose chains share a CU several at a time.  They do
-// not depend on how many systems a plan has, so a system's answer does not either.
-// Factorize and solve in FP64, one system, in us, with chains of 3 at every level against
-// these: n = 16, N = 2048: 141 -> 135; n = 32, 8192: 375 -> 333; n = 64, 2048: 509 -> 479,
-// 8192: 1125 -> 988; n = 128, 2048: 2310 -> 2100, 8192: 5563 -> 4886 (eight systems of 8192
-// blocks at n = 96: 18059 -> 16701).  From n = 64 on a level costs less than a block more in
-// each of its chains, so the later levels take chains of two and a base of four (n = 128, N =
-// 8192: 5082 with three and eight).  Below N = 1280 chains of three are as good or better
-// (n = 64, N = 512: 357, with seven 373), and need no more workspace.
-inline ChainLens auto_chain_lens(int N, int n) {
-  const int m = std::min(N / 256 - 1, n <= 32 ? 7 : n <= 64 ? 15 : 31);
-  if (m <= 3) return {3, 3, 8};
-  return n >= 64 ? ChainLens{m, 2, 4} : ChainLens{m, 3, 8};
-}
-
-// Full schedule: levels top first, the last one a single chain.
-// chain_len[k] > 0 fixes level k's chain length; other levels use `m_default`.
+// Full schedule: levels top first, the last one a single chain.  `chains` > 0 fixes the
+// number of chains of the first level, chain_len[k] > 0 the chain length of level k; other
+// levels use `m_default`.
 inline std::vector<LevelShape> auto_schedule(int N, const std::vector<int>& chain_len,
-                                             int m_default, int base_max) {
+                                             int m_default, int base_max, int chains = 0) {
   std::vector<LevelShape> out;
   int cur = N;
   size_t li = 0;
   while (cur > base_max && cur >= 3) {
     const int m = (li < chain_len.size() && chain_len[li] > 0) ? chain_len[li] : m_default;
-    LevelShape L = split_level(cur, std::max(1, m));
+    LevelShape L = split_level(cur, li == 0 && chains > 0 ? chains
+                                                          : chain_count(cur, std::max(1, m)));
     const int P = (int)L.seppos.size();
     out.push_back(std::move(L));
     cur = P;
@@ -155,6 +137,35 @@ inline std::vector<LevelShape> auto_schedule(int N, const std::vector<int>& chai
   }
   out.push_back(base_level(cur));
   return out;
+}
+
+// The schedule where no length is given.  Longer level-0 chains leave fewer separators (less
+// factor, panel and sweep work at every later level), as long as one system alone still has a
+// chain per CU: 256 chains, or, where they would be longer than a length from which the
+// chain's own latency costs more than the levels it saves (the smaller the blocks the earlier:
+// their chains share a CU several at a time), the nearest multiple of 256.  A multiple,
+// because a few chains more than that have the device to themselves while the others are done:
+// one FP32 system of n = 96, N = 5000, takes 1.05 ms with 256 chains of 19 and 1.56 with 263 of
+// 18 (chains of three: 1.23); n = 64, FP64: 0.74 with 256, 0.84 with 313 of 15.  Up to n = 32,
+// where a CU holds a dozen chains, the remainder does not matter and shorter chains are as
+// fast.  The schedule does not depend on how many systems a plan has, so a system's answer
+// does not either.
+// Factorize and solve in FP64, one system, in us, with chains of 3 at every level against
+// these: n = 16, N = 2048: 141 -> 135; n = 32, 8192: 375 -> 333; n = 64, 2048: 509 -> 479,
+// 8192: 1125 -> 988; n = 128, 2048: 2310 -> 2100, 8192: 5563 -> 4886 (eight systems of 8192
+// blocks at n = 96: 18059 -> 16701).  From n = 64 on a level costs less than a block more in
+// each of its chains, so the later levels take chains of two and a base of four (n = 128, N =
+// 8192: 5082 with three and eight).  Below N = 1280 chains of three are as good or better
+// (n = 64, N = 512: 357, with seven 373), and need no more workspace.
+inline std::vector<LevelShape> default_schedule(int N, int n) {
+  constexpr int CUS = 256;
+  if (N < 5 * CUS) return auto_schedule(N, {}, 3, 8);
+  const int longest = n <= 32 ? 7 : n <= 64 ? 15 : 31, per_cu = N / CUS;
+  int chains = CUS;
+  if (per_cu > longest + 1)
+    chains = n <= 32 ? chain_count(N, longest)
+                     : CUS * ((2 * per_cu + longest + 1) / (2 * (longest + 1)));
+  return n >= 64 ? auto_schedule(N, {}, 2, 4, chains) : auto_schedule(N, {}, 3, 8, chains);
 }
 
 inline std::vector<LevelShape> reference_schedule_levels(int N, int* n_use) {
