@@ -597,13 +597,17 @@ def build_smoother(data: BlockTriDiagData_batched, model) -> None:
     """Fill ``data.A_tensor``/``data.B_tensor`` (a single-system plan) with the
     smoother normal equations of ``model`` (``workloads.SmootherModel``), built on the
     device from F, H, Q^{-1}, R^{-1} (``bss_build_smoother``), asynchronously on the
-    current stream.  The blocks never cross PCIe."""
+    current stream.  The blocks never cross PCIe.  Refused while the stream is being
+    captured: a replay would read the model from host memory that is no longer its own."""
     if data.nsys != 1 or isinstance(data, BlockTriDiagData_group):
         raise ValueError("build_smoother fills a single-system plan")
     n = data.n
     if model.F.shape != (n, n):
         raise ValueError(f"model state size {model.F.shape} does not match n={n}")
     dev = data.device
+    with torch.cuda.device(dev):
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("build_smoother cannot be captured: its model comes from host memory")
     # column-major, one after the other: one copy to the device (four took 45 us each)
     parts = [np.asarray(M, dtype=np.float64).ravel(order="F")
              for M in (model.F, model.H, model.Qinv, model.Rinv)]
