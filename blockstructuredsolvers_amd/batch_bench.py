@@ -30,7 +30,7 @@ SIZES = (16, 32, 48, 64, 96, 128)
 # Level schedule of every system: level-0 chains of 15 blocks, 3 below, base 4.  On this
 # batch it is the fastest of the schedules tried, within 2% of each block size's own
 # best (MI355X, 512 systems: plain 7,451 -> 8,065 and mixed 8,077 -> 8,573 systems/s
-# against the library's default of chains of 3 and base 8).
+# against chains of 3 and base 8).
 SCHEDULE = dict(chain_len_levels=[15] + [3] * 15, base_max=4)
 
 

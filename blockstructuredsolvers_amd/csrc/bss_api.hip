@@ -1332,10 +1332,12 @@ int bss_factorize_solve(bss_plan_t p, void* stream) {
   p->info_valid = false;
   p->fb_active = p->fb_factored = false;
   // Up to n = 32 a level's sweep (4-6 us) takes less than the event record and the two waits
-  // that hand it to a second stream: everything in the caller's order was faster at every
-  // length (smoother requests, n = 16: 167 -> 143 us at N = 128, 241 -> 215 at N = 4096; n =
-  // 32: 213 -> 200 and 361 -> 349), and from n = 48 on slower (n = 64, N = 4096: 1044 ->
-  // 1113 us; n = 96, N = 300: 687 -> 724).
+  // that hand it to a second stream.  Second stream against the caller's order alone, us: n =
+  // 16, one system of 128 blocks 102 -> 71, of 8192 181 -> 150, eight of 300 in FP32 125 -> 73;
+  // n = 32, one of 128 141 -> 116.  Sweeps of many right-hand sides at n = 32 are long enough to
+  // gain a little from the second stream (8192 blocks, 16 right-hand sides: 369 -> 379 in FP64,
+  // 542 -> 580 mixed).  From n = 48 on it is the faster one (n = 64, N = 4096: 1044 -> 1113 us;
+  // n = 96, N = 300: 687 -> 724).
   const bool side = p->n > 32;
   if (side && !p->side_stream) {
     HIP_TRY(hipStreamCreateWithFlags(&p->side_stream, hipStreamNonBlocking));

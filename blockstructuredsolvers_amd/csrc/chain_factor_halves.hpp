@@ -13,7 +13,9 @@
 // SIMD's), and the eight diagonal tiles in turn between them.  Measured on MI355X, against
 // a kernel that kept only the triangle in LDS and staged every product's operands through
 // LDS in 16-row slices: 1024 chains of 15 blocks 7.20 -> 5.62 ms, 64 chains (less than
-// one a CU) 1.78 -> 1.30 ms.
+// one a CU) 1.78 -> 1.30 ms.  The three strips take 192 of a lane's 256 registers, and 87
+// values (188 bytes a lane) go to scratch all the same; the fences and the sums in memory below
+// keep it from more.
 #pragma once
 
 #include "chain_factor_strip.hpp"

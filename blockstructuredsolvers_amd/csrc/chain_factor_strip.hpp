@@ -15,8 +15,8 @@
 // current diagonal tile.
 //
 // What bounds it: per block the 4 to 8 diagonal tiles in turn (3.2K cycles each in FP64,
-// 2.5K in FP32, more beside other waves' MFMAs) and the products, about 60% of the MFMA
-// peak at n = 64.  Measured on MI355X, level-0 factorisation of 32 systems, N = 8192,
+// 2.5K in FP32, more beside other waves' MFMAs) and the products: at n = 64 in FP64 the matrix
+// cores are busy in 62% of the cycles and do 51% of their peak rate.  Measured on MI355X, level-0 factorisation of 32 systems, N = 8192,
 // n = 64, against the whole-block kernel before it: FP64 18.16 -> 12.2 ms, FP32 factors
 // of FP64 input with the fused forward sweep 9.13 -> 7.08 ms; 24 systems of n = 32, FP64:
 // 0.53 -> 0.29 ms; n = 48, FP32, 98 blocks in one chain: 0.90 -> 0.61 ms; n = 96, FP32
@@ -444,7 +444,8 @@ struct TileInverse {
 };
 
 // Waves per SIMD the registers are budgeted for (512 / this), from the workgroups that LDS
-// lets share a CU; every variant but n = 96 fits without spilling its strips.
+// lets share a CU.  Three variants spill: n = 96 FP64 (22 registers, 84 bytes a lane) and FP32
+// factors of FP64 input with the forward sweep at n = 96 (17, 40) and n = 48 (6, 28).
 template <typename T, int NB>
 constexpr int strip_waves_per_eu() {
   if (sizeof(T) == 8) return NB >= 48 ? 2 : 3;

@@ -299,7 +299,8 @@ struct TOps {
   }
 };
 
-// Several right-hand sides, up to 4 G.
+// Several right-hand sides, up to 4 G.  In FP64 at n = 128 the three panels of 64 registers and
+// the tiles do not quite fit: 3 registers go to scratch with G = 2, 38 (88 bytes a lane) with 4.
 template <typename T, int NB, int G>
 __global__ void __launch_bounds__(4 * NB) chain_forward_kernel(SolveLevelArgs p) {
   if (p.skip && *p.skip == 0) return;  // the whole workgroup leaves (uniform)

@@ -65,15 +65,17 @@ __global__ void __launch_bounds__(kRedThreads)
   berr[sys * nrhs + c] = den > 0.0 ? r / den : r;
 }
 
-// blocks per residual workgroup: at least 32, and at most 256 workgroups per system
-// (at N = 8192, two systems: two workgroups per CU, measured 3% faster than four with
-// 16 blocks each; 24 or 64 blocks were 30% slower)
+// blocks per residual workgroup: at least 32, and at most 256 workgroups per system.  An item
+// reads one B of its neighbour, and its four waves take its rows in turn.  Mixed solves with
+// resident factors, us, with 16, 32 and 64 blocks: n = 64, one system of 1024 191, 212, 260; 16
+// of 300 370, 366, 415; eight of 4096 1938, 1912, 1902; n = 128, 16 right-hand sides, 16 of
+// 300 2020, 1867, 2495; one of 128 670, 983, 1605.
 int blocks_per_item(int N) { return std::max(32, (N + 255) / 256); }
 
 // The first pass of a solve (x = 0, so r = d): d into the FP32 vector (the iterate is not
-// written: the first residual pass takes it as zero), and the item's per-column max |d_j| (as both the residual and the
-// right-hand-side maxima; the iterate maximum is 0).  Elementwise, with no block
-// window: one workgroup per residual work item, kInitThreads threads.
+// written: the first residual pass takes it as zero), and the item's per-column max |d_j| (as
+// both the residual and the right-hand-side maxima; the iterate maximum is 0).  Elementwise,
+// with no block window: one workgroup per residual work item, kInitThreads threads.
 constexpr int kInitThreads = 256;
 
 __global__ void __launch_bounds__(kInitThreads)

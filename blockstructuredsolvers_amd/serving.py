@@ -143,7 +143,7 @@ def _storage_order(blocks: np.ndarray) -> torch.Tensor:
 # options): level-0 chains of 31 blocks, 3 below, base 4.  On the served smoother stream
 # (n in {16, 32, 64}, N ~ U[128, 4096], all requests present at once) it raised the
 # served rate from 1,753 to 2,449 (plain) and 1,831 to 2,385 (mixed) systems/s against
-# the library default of chains of 3 and base 8.  ``solve_alone`` uses it too, so a
+# chains of 3 and base 8.  ``solve_alone`` uses it too, so a
 # served answer still equals the request solved alone.
 SERVE_SCHEDULE = {"chain_len_levels": [31] + [3] * 15, "base_max": 4}
 _SCHEDULE_KEYS = ("chain_len", "chain_len_levels", "base_max")

@@ -90,7 +90,9 @@ enum bss_option {
                                separator levels are re-factored in FP64 at the next
                                bss_solve or bss_info (which synchronise) */
   BSS_OPT_CHAIN_LEN = 3,    /* auto schedule: chain length for every level */
-  BSS_OPT_BASE_MAX = 4,     /* auto schedule: largest single-chain base level */
+  BSS_OPT_BASE_MAX = 4,     /* auto schedule: largest single-chain base level.  With neither
+                               this nor a chain length set both follow from N and n; with
+                               any of them set, lengths default to 3 and the base to 8 */
   BSS_OPT_PRESERVE_INPUT = 5, /* plain mode: 1 (default) = keep A and B unchanged, the
                                factors go to the plan's workspace (twice the A + B
                                bytes of workspace); 0 = overwrite A and B with the
@@ -214,11 +216,12 @@ int bss_solve(bss_plan_t plan, void* stream);
 /* bss_factorize followed by bss_solve, with the same results and the same state
  * afterwards (later bss_solve calls reuse the factors), for a caller whose d is
  * final before the factorisation starts.  Levels 0 and 1 are factored on `stream`;
- * then the first solve's forward sweeps (and, in mixed mode, its x = 0 residual pass)
- * run on a plan-owned stream: those of levels 0 and 1 beside the factorisation of
- * level 2, and each later level's as soon as that level is factored.  The side stream
- * is joined back into `stream` before the backward sweeps.  Returns what bss_solve
- * returns.  Replaces the reference's back-to-back
+ * then, for n > 32, the first solve's forward sweeps (and, in mixed mode, its x = 0
+ * residual pass) run on a plan-owned stream: those of levels 0 and 1 beside the
+ * factorisation of level 2, and each later level's as soon as that level is factored.  The
+ * side stream is joined back into `stream` before the backward sweeps.  For n <= 32 the
+ * sweeps are queued in the same places on `stream` itself, and there is no second stream.
+ * Returns what bss_solve returns.  Replaces the reference's back-to-back
  * factorize!(data); solve!(data) (src/gpu_batched.jl:184-259, as called in
  * test/test_rocm.jl:97-101); the reference has no combined call.  With BSS_OPT_GRAPH on,
  * or a single level, it is exactly bss_factorize then bss_solve. */
@@ -226,9 +229,8 @@ int bss_factorize_solve(bss_plan_t plan, void* stream);
 
 /* Factorize and solve one system in plain mode (dtype BSS_F64 or BSS_F32; A and B left
  * unchanged, solution in place in d) without allocating: no hipMalloc/hipFree and no
- * plan.  The same kernels, schedule (auto, chain length 3, base 8, 4 factor waves) and
- * results, bit for bit, as bss_factorize + bss_solve on a plan created with those
- * defaults.  Workspace and device tables come from a 64 MiB device array of the library
+ * plan.  The same kernels, schedule (auto, no length given) and results, bit for bit, as
+ * bss_factorize + bss_solve on a plan created with the defaults.  Workspace and device tables come from a 64 MiB device array of the library
  * (one per GPU, held until the process ends); systems whose workspace exceeds it (FP64:
  * about 550 blocks at n = 64, 2,200 at n = 32; BSS_Q_WORKSPACE_BYTES of a plan tells)
  * get BSS_E_ARG.  Set-up copies are ordered on `stream` (from pageable host memory,
