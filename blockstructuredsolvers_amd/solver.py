@@ -616,11 +616,16 @@ def build_smoother(data: BlockTriDiagData_batched, model) -> None:
         # elements starts its threads (n = 128 on 16 CPUs: 8.0 ms a request instead of 0.13)
         host = torch.empty(sum(p.size for p in parts), dtype=torch.float64, pin_memory=True)
         np.concatenate(parts, out=host.numpy())
-        F, H, Qi, Ri = torch.split(host.to(dev, non_blocking=True), [p.size for p in parts])
-        L.call("bss_build_smoother", data.n_user, n, model.H.shape[0], F.data_ptr(),
-               H.data_ptr(), Qi.data_ptr(), Ri.data_ptr(), data._a.data_ptr(),
-               data._b.data_ptr() if data._b.numel() else None, code, _stream_handle(dev))
-    data._model_tensors = (F, H, Qi, Ri)  # alive until the stream has used them
+        buf = host.to(dev, non_blocking=True)
+        del host  # the event of its return to the pool goes behind the copy, not the kernel
+        F = buf.data_ptr()
+        H = F + 8 * parts[0].size
+        Qi = H + 8 * parts[1].size
+        Ri = Qi + 8 * parts[2].size
+        L.call("bss_build_smoother", data.n_user, n, model.H.shape[0], F, H, Qi, Ri,
+               data._a.data_ptr(), data._b.data_ptr() if data._b.numel() else None, code,
+               _stream_handle(dev))
+    data._model_tensors = (buf,)  # alive until the stream has used it
 
 
 def reference_schedule(N: int):
