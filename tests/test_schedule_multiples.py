@@ -9,7 +9,7 @@ from chain_emulator import plan_levels
 @pytest.mark.parametrize("N", [1280, 1281, 1700, 2047, 2048, 2049, 3000, 4095, 4097, 5000, 6144,
                                6500, 8192, 8193, 9000, 12288, 20000, 40000])
 @pytest.mark.parametrize("n", [48, 64, 96, 128])
-def test_whole_rounds(N, n):
+def test_multiples_of_the_cus(N, n):
     _, levels = plan_levels(N, n)
     lens = [c[1] for c in levels[0][1]]
     assert len(lens) % 256 == 0
