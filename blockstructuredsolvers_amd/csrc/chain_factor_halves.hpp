@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(4 * NB) __attribute__((amdgpu_waves_per_eu(2))
   const int w = wave_id();
   const int l = lane_id(), lr = l & 15, lk = l >> 4;
   const int so = I::own_slot(), sa = I::a_slot();
-  const TileInverse<T, NB> inv{As, Rs, Es, Is, &fail, w, so, sa};
+  const TileInverse<T, NB, true> inv{As, Rs, Es, Is, &fail, w, so, sa};
   const int lcol = lr * NB + I::row(lk, 0);  // this lane's elements of a tile in HBM
 
   // keeps the scheduler from loading more than two steps' operands ahead (they would spill)

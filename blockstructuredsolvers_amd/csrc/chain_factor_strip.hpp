@@ -185,17 +185,16 @@ __device__ __attribute__((always_inline)) inline double write_lane(double x, dou
 // Elimination steps of the 16x16 tile.  Every lane holds a column v[0..15]: in the even
 // 16-lane rows column c = lane % 16 of A, in the odd ones column c of the identity, which
 // becomes that of E.  Step J subtracts A[J][r] / A[J][J] times row J from the rows r > J
-// of both at once: m (row J of A in every 16-lane row) supplies the multipliers by DPP, f
-// (row J, negated) is the lane's own factor.  Each of them takes 1 / sqrt of the pivot: 1 /
-// A[J][J] on one of them would be denormal for a pivot in the top binades (FP32's rcp returns
-// zero above 2^126), and takes 1% off a small FP64 system (n = 32, 100 blocks: 104.5 us, this
-// 105.7; powers of two formed on the scalar unit 110.5, tiles with such a diagonal scaled
-// under a branch 107.6).  One FMA per row serves A and E (the same steps on separate A and E
-// registers take twice the FMAs, which a wave shares its SIMD's issue slots for with the other
-// waves' MFMAs).  Only the upper part of A is read.  The scaling by 1 / sqrt of the pivots
-// (gathered in pv) is left to the end.  The next step's pivot chain is interleaved with this
-// step's rows by hand: sched_barrier keeps the order.
-template <int J>
+// of both at once: m (row J of A in every 16-lane row) supplies the multipliers by DPP,
+// f = -v[J] / A[J][J] is the lane's own factor.  One FMA per row serves A and E (the same
+// steps on separate A and E registers take twice the FMAs, which a wave shares its SIMD's
+// issue slots for with the other waves' MFMAs).  Only the upper part of A is read.  The
+// scaling by 1 / sqrt of the pivots (gathered in pv) is left to the end.  The next step's
+// pivot chain is interleaved with this step's rows by hand: sched_barrier keeps the order.
+// WIDE: m and f have 1 / sqrt of the pivot each, for any pivot: 1 / A[J][J] on f alone is
+// denormal for a pivot in the top binades (FP32's rcp returns zero above 2^126), and with a
+// large E overflows for one in the bottom binades.
+template <int J, bool WIDE>
 __device__ __attribute__((always_inline)) inline void elim_step(double (&v)[16], double m,
                                                                 double f, double& pv) {
   if constexpr (J < 15) {
@@ -210,16 +209,17 @@ __device__ __attribute__((always_inline)) inline void elim_step(double (&v)[16],
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 3, J + 4>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const double y = __builtin_amdgcn_rsq(p);  // about 2^-24; third-order step below
+    // about 2^-24; third-order step below
+    const double y = WIDE ? __builtin_amdgcn_rsq(p) : __builtin_amdgcn_rcp(p);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 4, J + 6>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const double py = p * y;
+    const double py = WIDE ? p * y : p;
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 6, J + 7>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
     const double e = fma(-py, y, 1.0), g = v[J + 1] * y;
-    mn *= y;
+    if constexpr (WIDE) mn *= y;
     pv = write_lane<J + 1>(pv, p);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 7, J + 8>(v, m, f);
@@ -231,10 +231,10 @@ __device__ __attribute__((always_inline)) inline void elim_step(double (&v)[16],
     const double fn = fma(-g, t, -g);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 9, 16>(v, m, f);
-    elim_step<J + 1>(v, mn, fn, pv);
+    elim_step<J + 1, WIDE>(v, mn, fn, pv);
   }
 }
-template <int J>
+template <int J, bool WIDE>
 __device__ __attribute__((always_inline)) inline void elim_step(float (&v)[16], float m, float f,
                                                                 float& pv) {
   if constexpr (J < 15) {
@@ -249,28 +249,41 @@ __device__ __attribute__((always_inline)) inline void elim_step(float (&v)[16], 
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 3, J + 4>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
-    const float y = __builtin_amdgcn_rsqf(p);  // 1 ulp, as the sweep's other roundings
+    // 1 ulp, as the sweep's other roundings
+    const float y = WIDE ? __builtin_amdgcn_rsqf(p) : __builtin_amdgcn_rcpf(p);
     pv = write_lane<J + 1>(pv, p);
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 4, J + 7>(v, m, f);
     __builtin_amdgcn_sched_barrier(0);
     const float fn = -(v[J + 1] * y);
-    mn *= y;
+    if constexpr (WIDE) mn *= y;
     __builtin_amdgcn_sched_barrier(0);
     fmac_rows<J + 7, 16>(v, m, f);
-    elim_step<J + 1>(v, mn, fn, pv);
+    elim_step<J + 1, WIDE>(v, mn, fn, pv);
   }
 }
-// the first step's m and f from row 0
-__device__ inline void first_row(double x, double p, double& m, double& f) {
-  const double y = __builtin_amdgcn_rsq(p), e = fma(-(p * y), y, 1.0), g = x * y;
-  m = even_rows(x) * y;
-  f = fma(-g, fma(e, e, e), -g);
+template <bool WIDE>
+__device__ __attribute__((always_inline)) inline void eliminate(double (&v)[16], double& pv) {
+  const double p = read_lane(v[0], 0);
+  const double y = WIDE ? __builtin_amdgcn_rsq(p) : __builtin_amdgcn_rcp(p);
+  const double e = fma(-(WIDE ? p * y : p), y, 1.0), g = v[0] * y;
+  pv = write_lane<0>(1.0, p);
+  elim_step<0, WIDE>(v, WIDE ? even_rows(v[0]) * y : even_rows(v[0]), fma(-g, fma(e, e, e), -g),
+                     pv);
 }
-__device__ inline void first_row(float x, float p, float& m, float& f) {
-  const float y = __builtin_amdgcn_rsqf(p);
-  m = even_rows(x) * y;
-  f = -(x * y);
+template <bool WIDE>
+__device__ __attribute__((always_inline)) inline void eliminate(float (&v)[16], float& pv) {
+  const float p = read_lane(v[0], 0);
+  const float y = WIDE ? __builtin_amdgcn_rsqf(p) : __builtin_amdgcn_rcpf(p);
+  pv = write_lane<0>(1.0f, p);
+  elim_step<0, WIDE>(v, WIDE ? even_rows(v[0]) * y : even_rows(v[0]), -(v[0] * y), pv);
+}
+// whether x is in [2^-1000, 2^1000) (FP32: [2^-100, 2^100))
+__device__ inline bool mid_range(double x) {
+  return (unsigned)__double2hiint(x) - (23u << 20) < (2000u << 20);
+}
+__device__ inline bool mid_range(float x) {
+  return __float_as_uint(x) - (27u << 23) < (200u << 23);
 }
 template <int R, typename T>
 __device__ __attribute__((always_inline)) inline void scale_rows(T (&v)[16], T s) {
@@ -283,27 +296,43 @@ __device__ __attribute__((always_inline)) inline void scale_rows(T (&v)[16], T s
 // Cholesky + inverse of the symmetric 16x16 tile with image `at` (upper part): the image of
 // Uinv = U^-1 (strict lower part exact zeros) to `ut` (may be `at`), the image of E = Uinv^T
 // to `et`; `eye` is the image of the identity.  Returns false if a pivot was not positive.
-template <typename T>
+// One unsigned comparison of the exponents finds the pivots that are not positive and those
+// whose reciprocal may leave the exponent range (the first of either is itself right); for the
+// latter the tile is done again, WIDE.  WIDE in every tile takes 1% off a small FP64 system (n
+// = 32, 100 blocks: 104.5 -> 105.7 us; this 105.0), and loses 2% of the accuracy of FP64
+// tiles.  ALWAYS_WIDE: the same, for a kernel in which the second try's registers spill (FP64
+// at n = 128, 16 right-hand sides: 5.24 -> 5.24 ms, with the second try 5.30 to 5.51).
+template <typename T, bool ALWAYS_WIDE>
 __device__ __attribute__((always_inline)) inline bool diag_img(const T* at, T* ut, T* et,
                                                                const T* eye) {
   typedef Img<T> I;
   const int c = opaque_v(lane_id() & 15);
-  const bool odd = (lane_id() >> 4) & 1;
-  T v[16];
-  const T* src = odd ? eye : at;
+  T v[16], pv;
+  auto load = [&](int c) {
+    const T* src = (lane_id() >> 4) & 1 ? eye : at;
 #pragma unroll
-  for (int g = 0; g < 16 / I::VEC; ++g) {
-    const auto t = *(const typename I::vec_t*)(src + I::off(I::VEC * g, c));
+    for (int g = 0; g < 16 / I::VEC; ++g) {
+      const auto t = *(const typename I::vec_t*)(src + I::off(I::VEC * g, c));
 #pragma unroll
-    for (int q = 0; q < I::VEC; ++q) v[I::VEC * g + q] = t[q];
+      for (int q = 0; q < I::VEC; ++q) v[I::VEC * g + q] = t[q];
+    }
+  };
+  load(c);
+  eliminate<ALWAYS_WIDE>(v, pv);
+  T s = rsqrt_nr(pv);
+  bool ok = true;
+  if (__builtin_amdgcn_ballot_w64(!mid_range(pv)) != 0) {
+    if constexpr (!ALWAYS_WIDE) {
+      if (__builtin_amdgcn_ballot_w64(pv > T(0) && !mid_range(pv)) != 0) {
+        load(opaque_v(lane_id() & 15));
+        eliminate<true>(v, pv);
+        s = rsqrt_nr(pv);
+      }
+    }
+    ok = __builtin_amdgcn_ballot_w64(!(pv > T(0))) == 0;
   }
-  const T p = read_lane(v[0], 0);
-  T pv = write_lane<0>(T(1), p);
-  T m, f;
-  first_row(v[0], p, m, f);
-  elim_step<0>(v, m, f, pv);
   __builtin_amdgcn_sched_barrier(0);
-  scale_rows<0>(v, even_rows(rsqrt_nr(pv)));
+  scale_rows<0>(v, even_rows(s));
   if ((lane_id() >> 4) == 1) {  // E[r][c] = Uinv[c][r] in v[r]
 #pragma unroll
     for (int r = 0; r < 16; ++r) ut[I::off(c, r)] = v[r];
@@ -315,7 +344,7 @@ __device__ __attribute__((always_inline)) inline bool diag_img(const T* at, T* u
       *(typename I::vec_t*)(et + I::off(I::VEC * g, c)) = t;
     }
   }
-  return __builtin_amdgcn_ballot_w64(!(pv > T(0))) == 0;
+  return ok;
 }
 
 // N tiles, one below the other, from consecutive images in LDS to HBM (column-major, leading
@@ -352,7 +381,7 @@ __device__ __attribute__((always_inline)) inline void put_tiles(BSS_GLOBAL T* g,
 // k is never rewritten and one barrier per diagonal tile is enough; with a row-scaling
 // phase and its barrier the FP64 factorisation at n = 64 took 13.6 ms where it takes 12.2.
 // `extra(k)` is the caller's own work in window k.
-template <typename T, int NB>
+template <typename T, int NB, bool ALWAYS_WIDE = false>
 struct TileInverse {
   typedef Img<T> I;
   typedef typename I::tile_t tile_t;
@@ -401,7 +430,7 @@ struct TileInverse {
           }
           I::store(up(w, w), so, acc);
         }
-        if (!diag_img<T>(up(w, w), up(w, w), ed(w), Is) && lane_id() == 0) *fail = 1;
+        if (!diag_img<T, ALWAYS_WIDE>(up(w, w), up(w, w), ed(w), Is) && lane_id() == 0) *fail = 1;
       } else if (k >= 0) {
         const tile_t x = I::load(up(k, k), sa);
         const int u = w - (w > k + 1 ? 1 : 0);
